@@ -4,4 +4,5 @@
 #include "prim.hip"
 #include "attn.hip"
 #include "gemm.hip"
+#include "tile.hip"
 #include "rows.hip"

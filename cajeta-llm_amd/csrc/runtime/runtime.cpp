@@ -322,6 +322,29 @@ GemvPlan plan_gemv(int type, int64_t rows, int64_t cols, int target, int pro, in
 
 bool gemm_supported(int type) { return type == CJ_Q8_0 || type == CJ_Q4_K || type == CJ_Q6_K; }
 
+// The K-quants' 64-row × 128-column tile kernel (tile.hip) takes about
+// 2.05 us a 256-element block and round of tiles over the CUs, however full
+// the tiles are. Its lines, measured on 256 CUs (us, 4096 columns of weights
+// unless named; other kernel → tile kernel):
+//  - Q4_K: where the 64 × 32 tiles of the other kernel are more than one a CU
+//    for each round (4096 × 128: 31.5 → 34.2 stays; 6144 × 96: 43.9 → 33.3;
+//    4096 × 512: 75.9 → 34.2; 28672 × 17, two rounds: 45.8 → 65.9 stays,
+//    × 33: 84.2 → 66.8);
+//  - Q6_K: where rows × columns (in 16s) pass 1200 a CU for each round, the
+//    other kernel's 30 us (2048 × 128: 29.6 → 32.7 stays; 6144 × 64: 42.5 →
+//    32.4; 28672 × 17: 81 → 64; 4096 × 512: 209 → 35.5).
+static bool gemm_tiled(const cj_gemv_args &a, int64_t &wgs) {
+    if ((a.type != CJ_Q4_K && a.type != CJ_Q6_K) || a.batch <= 16) return false;
+    // its copies into LDS move aligned 16-byte words
+    if ((((uintptr_t)a.w | (uintptr_t)a.xp | (uintptr_t)a.xp_stride | (uintptr_t)a.row_bytes) & 15) != 0) return false;
+    const int64_t cus = std::max(1, g.cus), gx = ((int64_t)a.batch + 127) / 128, gy = (a.rows + 63) / 64;
+    const int64_t rounds = (gx * gy + cus - 1) / cus;
+    wgs = gx * (gy >= 8 ? (gy + 7) / 8 * 8 : gy);
+    if (wgs > 0x7fffffff || (a.type == CJ_Q4_K && gy > 65535)) return false;
+    if (a.type == CJ_Q4_K) return gy * (((int64_t)a.batch + 31) / 32) > cus * rounds;
+    return a.rows * (((int64_t)a.batch + 15) / 16 * 16) > 1200 * cus * rounds;
+}
+
 // Two kernels, chosen by shape. The tiled kernel (4 waves a 64-row ×
 // 16·NT-column tile over LDS-staged packs) when the row blocks and column
 // tiles make at least 256 workgroups (a CU's worth each) — tall projections,
@@ -344,6 +367,11 @@ int run_gemm(const cj_gemv_args &a) {
         const int rw = (a.rows + 15) / 16 * cgroups >= 2 * (int64_t)std::max(1, g.cus) ? 4 : 2;
         snprintf(name, sizeof name, "cj_gemm_q40_r%d_c4", rw);
         return launch2(name, (uint32_t)((a.rows + 4 * rw - 1) / (4 * rw)), (uint32_t)cgroups, 256, 0, a);
+    }
+    int64_t wgs = 0;
+    if (gemm_tiled(a, wgs)) {
+        if (a.cols % 256) return fail(CJ_ERR_ARG, "gemm: K-quant rows are whole 256-element blocks");
+        return launch(a.type == CJ_Q4_K ? "cj_gemm_t_q4k" : "cj_gemm_t_q6k", (uint32_t)wgs, 512, 0, a);
     }
     if (a.type == CJ_Q6_K) {
         // many-column GEMV (4 or 8 columns a grid row; its LDS fixed: a
@@ -419,7 +447,7 @@ int32_t cj_init(int32_t device) {
         "cj_attn_combine_h64", "cj_attn_combine_h128", "cj_attn_fused_h64", "cj_attn_fused_h128",
         "cj_attn_merge", "cj_attn_merge_q", "cj_moe_group", "cj_argmax_pick", "cj_qkprep", "cj_zero", "cj_moe_route", "cj_router_topk",
         "cj_gemm_q80_n2", "cj_gemm_q4k_n2", "cj_gemm_q80_n4", "cj_gemm_q6k_c4", "cj_gemm_q6k_c8", "cj_gemm_q6k_m16",
-        "cj_gemm_sk_q80_n1", "cj_gemm_sk_q80_n2", "cj_gemm_sk_q4k_n1",
+        "cj_gemm_sk_q80_n1", "cj_gemm_sk_q80_n2", "cj_gemm_sk_q4k_n1", "cj_gemm_t_q4k", "cj_gemm_t_q6k",
         "cj_rows_embed", "cj_rows_qkv", "cj_rows_glu", "cj_rows_argmax", "cj_rows_pick",
         "cj_attn_split_rows_h128_g4", "cj_attn_split_rows_h128_g8", "cj_attn_merge_rows",
         "cj_attn_prefill_h128_g1", "cj_attn_prefill_h128_g2", "cj_attn_prefill_h128_g4", "cj_attn_prefill_h128_g8",

@@ -676,3 +676,44 @@ def test_allocating_argmax_refuses_a_graph_capture(gpu):
     gpu.native.check(lib.cj_graph_free(gh), "graph free")
     gpu.native.check(lib.cj_argmax_row(tb.h, 0, v.h, 5000), "argmax")
     assert tb.download(np.int32, 1)[0] == 4999
+
+
+@pytest.mark.parametrize("name,ty", [("q4_k", 12), ("q6_k", 14)])
+@pytest.mark.parametrize("rows,cols,ncols", [(4160, 256, 130), (4161, 1280, 129), (8200, 512, 127), (2050, 2304, 300),
+                                             (40, 768, 30000), (16448, 1024, 33)])
+def test_matmul_tile_kernels(gpu, O, name, ty, rows, cols, ncols):
+    """Shapes that take the 64-row × 128-column tile kernels (more tiles than
+    a CU's worth of the others'), off the tile's edges, one block to nine:
+    every column checked bit for bit against the oracle's one-column product.
+    Row 0 and column 0 hold the largest codes and scales, so their integer
+    sums reach their bounds."""
+    say("matmul tile", name, rows, cols, ncols)
+    rng = np.random.default_rng(rows + cols * 3 + ncols + ty)
+    be, bb = O.BLOCK[ty]
+    raw = rand_blocks(O, ty, rows * cols // be, rng).reshape(rows, cols // be, bb).copy()
+    if ty == O.Q4_K:
+        raw[0, :, 4:] = 0xFF                       # every scale, min and code at its largest
+    else:
+        raw[0, :, :192] = 0                        # every code −32
+        raw[0, :, 192:208] = 0x80                  # every scale −128
+    lib = gpu.native.lib()
+    w = gpu.Buffer(lib.cj_prepared_row_bytes(ty, cols) * rows)
+    src = gpu.Buffer.of(raw.reshape(-1))
+    gpu.native.check(lib.cj_prepare_weight(w.h, src.h, ty, rows, cols), "prepare")
+    distinct = min(ncols, 40)                      # later columns repeat them
+    x = rng.standard_normal((distinct, cols)).astype(np.float32)
+    x[0] = 1.0
+    stride = cols // 256 * 320 + 32
+    packs = np.zeros((ncols, stride), np.uint8)
+    for c in range(distinct):
+        packs[c, :stride - 32] = O.q8k_pack(x[c])
+    packs[:] = packs[np.arange(ncols) % distinct]
+    refs = np.stack([O.matvec_packed(ty, raw.reshape(-1), rows, cols, packs[c, :stride - 32]) for c in range(distinct)])
+    xb, y = gpu.Buffer.of(packs.reshape(-1)), gpu.Buffer(ncols * rows * 4)
+    gpu.native.check(lib.cj_matmul(ty, y.h, w.h, xb.h, rows, cols, ncols, stride, rows, 0, 0), "matmul")
+    got = y.download(np.float32, ncols * rows).reshape(ncols, rows)
+    for c in range(ncols):
+        assert np.array_equal(got[c].view(np.uint32), refs[c % distinct].view(np.uint32)), \
+            "%s column %d: %d rows differ" % (name, c, int((got[c] != refs[c % distinct]).sum()))
+    for b in (w, src, xb, y):
+        b.free()
