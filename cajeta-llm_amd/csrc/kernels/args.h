@@ -135,6 +135,9 @@ typedef struct { float *a; const float *b; int64_t n; } cj_add_args;
 
 typedef struct { void *dst; const void *src; int64_t n16; } cj_copy_args;
 
+// out (pinned host memory): {lowest entry, highest entry, ticket}, the ticket last
+typedef struct { const int32_t *tab; int32_t *out; int64_t n; int32_t ticket; } cj_page_args;
+
 typedef struct {
     float *q, *k; const float *v;
     uint16_t *kc, *vc;

@@ -146,6 +146,37 @@ extern "C" __global__ void __launch_bounds__(256) cj_copy(cj_copy_args a) {
         ((uint4 *)a.dst)[i] = ((const uint4 *)a.src)[i];
 }
 
+// The lowest and highest entry of a page table, to host memory that the
+// caller polls for the ticket: what an attend checks before it launches. A
+// copy of the table to the host waited for twice the copy engine's latency
+// and staged pageable memory (bound by latency; one attend with its QK prep
+// at 2049 positions 95 us a pass with the copies, 72 us with this; 76 → 52 at 4097 positions, head size 64).
+extern "C" __global__ void __launch_bounds__(256) cj_page_span(cj_page_args a) {
+    __shared__ int32_t lo[256], hi[256];
+    const int t = threadIdx.x;
+    int32_t l = a.tab[0], h = l;
+    for (int64_t i = t; i < a.n; i += 256) {
+        const int32_t v = a.tab[i];
+        l = min(l, v);
+        h = max(h, v);
+    }
+    lo[t] = l;
+    hi[t] = h;
+    __syncthreads();
+    for (int s = 128; s > 0; s >>= 1) {
+        if (t < s) {
+            lo[t] = min(lo[t], lo[t + s]);
+            hi[t] = max(hi[t], hi[t + s]);
+        }
+        __syncthreads();
+    }
+    if (t == 0) {
+        a.out[0] = lo[0];
+        a.out[1] = hi[0];
+        __hip_atomic_store(a.out + 2, a.ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 // ------------------------------------------------------------------ glu
 
 // One workgroup per 256-wide block: out = act(g)·u, then (optionally) that

@@ -5,6 +5,7 @@
 #include "rt.h"
 #include <dlfcn.h>
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -38,6 +39,9 @@ struct Ctx {
     int64_t hbm = 0;
     int64_t lds = 0;
     std::map<int, void *> scratch_at;   // device → address of `scratch` on it
+    int32_t *span = nullptr;            // pinned {lowest, highest, ticket} of the last page table checked
+    uint32_t span_ticket = 0;
+    std::mutex span_mu;
 };
 Ctx g;
 thread_local std::string g_err;
@@ -188,6 +192,42 @@ int launch_raw(const char *name, uint32_t grid, uint32_t block, uint32_t lds, co
 }
 
 uint64_t launch_count() { return g_launches; }
+
+// The lowest and highest of the n page-table entries at `tab`, read in stream
+// order (entries that queued work writes are seen). A kernel writes them to
+// pinned memory and the host polls for its ticket, which costs a launch and a
+// store over the bus; the table's copy to the host, which a capturing stream
+// still takes (and refuses, as before), costs a copy engine's round trip and
+// a stream synchronize.
+static int page_span(const void *tab, int64_t n, int32_t &lo, int32_t &hi) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    (void)hipStreamIsCapturing(g.stream, &cap);
+    if (cap == hipStreamCaptureStatusNone && g.span && has_kernel("cj_page_span")) {
+        std::lock_guard<std::mutex> lk(g.span_mu);
+        const int32_t ticket = (int32_t)++g.span_ticket;
+        cj_page_args a{(const int32_t *)tab, g.span, n, ticket};
+        if (int rc = launch("cj_page_span", 1, 256, 0, a)) return rc;
+        const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(5);
+        for (int spin = 0;; spin++) {
+            if (__atomic_load_n(g.span + 2, __ATOMIC_ACQUIRE) == ticket) break;
+            if ((spin & 255) == 255 && std::chrono::steady_clock::now() > until) {
+                // long work is queued ahead, or the device failed: wait as the copy would
+                CJ_HIP(hipStreamSynchronize(g.stream));
+                if (__atomic_load_n(g.span + 2, __ATOMIC_ACQUIRE) != ticket) return fail(CJ_ERR_HIP, "page table check did not report");
+                break;
+            }
+        }
+        lo = g.span[0];
+        hi = g.span[1];
+        return CJ_OK;
+    }
+    std::vector<int32_t> v((size_t)n);
+    CJ_HIP(hipMemcpyAsync(v.data(), tab, (size_t)n * 4, hipMemcpyDeviceToHost, g.stream));
+    CJ_HIP(hipStreamSynchronize(g.stream));
+    lo = *std::min_element(v.begin(), v.end());
+    hi = *std::max_element(v.begin(), v.end());
+    return CJ_OK;
+}
 
 // ------------------------------------------------------------------ GEMV
 
@@ -442,7 +482,7 @@ int32_t cj_init(int32_t device) {
         "cj_gemv_q40b_r2", "cj_gemv_q40b_r4", "cj_gemm_q40_r2_c4", "cj_gemm_q40_r4_c4",
         "cj_gemv_mxfp4", "cj_gemv_f32", "cj_gemv_mxfp4_r32", "cj_gemv_f32_r32", "cj_gemv_mxfp4_r1", "cj_gemv_f32_r1",
         "cj_moe_combine", "cj_moe_combine_norm",
-        "cj_pack", "cj_norm_pack", "cj_norm_pack_rows", "cj_copy", "cj_glu", "cj_add", "cj_dequant", "cj_prepare", "cj_embed", "cj_argmax",
+        "cj_pack", "cj_norm_pack", "cj_norm_pack_rows", "cj_copy", "cj_page_span", "cj_glu", "cj_add", "cj_dequant", "cj_prepare", "cj_embed", "cj_argmax",
         "cj_attn_split_h128_g4", "cj_attn_split_h128_g8", "cj_attn_scores_h64", "cj_attn_scores_h128",
         "cj_attn_combine_h64", "cj_attn_combine_h128", "cj_attn_fused_h64", "cj_attn_fused_h128",
         "cj_attn_merge", "cj_attn_merge_q", "cj_moe_group", "cj_argmax_pick", "cj_qkprep", "cj_zero", "cj_moe_route", "cj_router_topk",
@@ -493,6 +533,9 @@ int32_t cj_init(int32_t device) {
                     if (hipModuleGetFunction(&f, g.module, k.c_str()) == hipSuccess) g.fns[k] = f;
                 }
     CJ_HIP(hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking));
+    if (hipHostMalloc((void **)&g.span, 64, 0) != hipSuccess) return fail(CJ_ERR_HIP, "pinned page-table check");
+    memset(g.span, 0, 64);
+    g.span_ticket = 0;
     g.device = device;
     void *sp = nullptr;
     int rc = scratch_here(&sp);   // the allocation-free entry point's scratch, set up with the device current
@@ -511,6 +554,8 @@ int32_t cj_shutdown(void) {
     }
     for (auto p : ps) (void)hipFree((void *)p);
     (void)hipStreamDestroy(g.stream);
+    if (g.span) (void)hipHostFree(g.span);
+    g.span = nullptr;
     (void)hipModuleUnload(g.module);
     g.module = nullptr;
     g.fns.clear();
@@ -794,9 +839,8 @@ int32_t cj_qk_prep(int64_t q, int64_t k, int64_t v, int64_t kcache, int64_t vcac
         !in_buffer(dptr(rope), ((int64_t)pos + 1) * head_dim * 4) ||
         (norm && (!in_buffer(dptr(qw), head_dim * 4) || !in_buffer(dptr(kw), head_dim * 4))))
         return fail(CJ_ERR_ARG, "cj_qk_prep: a buffer is smaller than the shapes need");
-    int32_t pg = 0;
-    CJ_HIP(hipMemcpyAsync(&pg, dptr(pgtab + 4 * (pg_base + page)), 4, hipMemcpyDeviceToHost, g.stream));
-    CJ_HIP(hipStreamSynchronize(g.stream));
+    int32_t pg = 0, hi = 0;
+    if (int32_t rc = page_span(dptr(pgtab + 4 * (pg_base + page)), 1, pg, hi)) return rc;
     const int64_t need = (((int64_t)pg + 1) * n_kv * 64) * head_dim * 2;
     if (pg < 0 || !in_buffer(dptr(kcache), need) || !in_buffer(dptr(vcache), need))
         return fail(CJ_ERR_CAPACITY, "cj_qk_prep: page %d outside the K/V planes", pg);
@@ -825,14 +869,9 @@ int32_t cj_attend(int64_t part, int64_t out, int64_t q, int64_t kcache, int64_t 
         (out && !in_buffer(dptr(out), (int64_t)n_q * head_dim * 4)) ||
         (split && out && !in_buffer(dptr(counters), (int64_t)n_kv * 4)))
         return fail(CJ_ERR_ARG, "cj_attend: a buffer is smaller than the shapes need");
-    std::vector<int32_t> tab((size_t)pages);
-    CJ_HIP(hipMemcpyAsync(tab.data(), dptr(pgtab + 4 * pg_base), (size_t)pages * 4, hipMemcpyDeviceToHost, g.stream));
-    CJ_HIP(hipStreamSynchronize(g.stream));
-    int32_t maxpg = 0;
-    for (int32_t p : tab) {
-        if (p < 0) return fail(CJ_ERR_ARG, "cj_attend: negative page in the table");
-        maxpg = std::max(maxpg, p);
-    }
+    int32_t minpg = 0, maxpg = 0;
+    if (int32_t rc = page_span(dptr(pgtab + 4 * pg_base), pages, minpg, maxpg)) return rc;
+    if (minpg < 0) return fail(CJ_ERR_ARG, "cj_attend: negative page in the table");
     const int64_t need = (((int64_t)maxpg + 1) * n_kv * 64) * head_dim * 2;
     if (!in_buffer(dptr(kcache), need) || !in_buffer(dptr(vcache), need))
         return fail(CJ_ERR_ARG, "cj_attend: page %d outside the K/V planes", maxpg);
@@ -987,14 +1026,9 @@ int32_t cj_attn_scores(int64_t scores, int64_t q, int64_t kcache, int64_t pgtab,
     if (!in_buffer(dptr(pgtab + 4 * (int64_t)pg_base), pages * 4) || !in_buffer(dptr(q), (int64_t)n_q * head_dim * 4) ||
         !in_buffer(dptr(scores), (int64_t)n_q * count * 4))
         return fail(CJ_ERR_ARG, "cj_attn_scores: a buffer is smaller than the shapes need");
-    std::vector<int32_t> tab((size_t)pages);
-    CJ_HIP(hipMemcpyAsync(tab.data(), dptr(pgtab + 4 * (int64_t)pg_base), (size_t)pages * 4, hipMemcpyDeviceToHost, g.stream));
-    CJ_HIP(hipStreamSynchronize(g.stream));
-    int32_t maxpg = 0;
-    for (int32_t p : tab) {
-        if (p < 0) return fail(CJ_ERR_ARG, "cj_attn_scores: negative page in the table");
-        maxpg = std::max(maxpg, p);
-    }
+    int32_t minpg = 0, maxpg = 0;
+    if (int32_t rc = page_span(dptr(pgtab + 4 * (int64_t)pg_base), pages, minpg, maxpg)) return rc;
+    if (minpg < 0) return fail(CJ_ERR_ARG, "cj_attn_scores: negative page in the table");
     if (!in_buffer(dptr(kcache), (((int64_t)maxpg + 1) * n_kv * 64) * head_dim * 2))
         return fail(CJ_ERR_ARG, "cj_attn_scores: page %d outside the K plane", maxpg);
     cj_attn_args a{};

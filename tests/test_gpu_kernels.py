@@ -717,3 +717,40 @@ def test_matmul_tile_kernels(gpu, O, name, ty, rows, cols, ncols):
             "%s column %d: %d rows differ" % (name, c, int((got[c] != refs[c % distinct]).sum()))
     for b in (w, src, xb, y):
         b.free()
+
+
+@pytest.mark.parametrize("pages", [1, 2, 255, 256, 257, 700])
+def test_page_table_checks(gpu, O, pages):
+    """A page outside the planes or below zero is refused wherever in the
+    table it stands, also when work queued just before writes it, and a good
+    table is accepted right after: the check reads the table in stream order."""
+    say("page table checks", pages)
+    lib = gpu.native.lib()
+    nq, nkv, hd, count = 2, 1, 64, pages * 64
+    planes = 3                                           # pages 0..2 exist
+    kc, vc = gpu.Buffer(planes * nkv * 64 * hd * 2), gpu.Buffer(planes * nkv * 64 * hd * 2)
+    kc.zero(); vc.zero()
+    q, out = gpu.Buffer(nq * hd * 4), gpu.Buffer(nq * hd * 4)
+    part = gpu.Buffer(nq * count * 4)
+    q.zero()
+    words = (pages + 3) // 4 * 4
+    tab = gpu.Buffer(words * 4)
+
+    def attend():
+        return lib.cj_attend(part.h, out.h, q.h, kc.h, vc.h, tab.h, 0, 0, nq, nkv, hd, count, 0, 512, 0.125)
+
+    good = np.zeros(words, np.int32)
+    good[:pages] = np.arange(pages) % planes
+    gb = gpu.Buffer.of(good)
+    for at in sorted({0, pages // 2, pages - 1}):
+        for v in (planes, -1):
+            bad = good.copy()
+            bad[at] = v
+            bb = gpu.Buffer.of(bad)
+            gpu.native.check(lib.cj_buf_copy(tab.h, bb.h, words * 4), "copy")
+            assert attend() == -1 and ("negative" if v < 0 else "outside") in gpu.native.last_error()
+            assert lib.cj_attn_scores(part.h, q.h, kc.h, tab.h, 0, nq, nkv, hd, count, 0, 0.125) == -1
+            gpu.native.check(lib.cj_buf_copy(tab.h, gb.h, words * 4), "copy")
+            assert attend() == 0
+            gpu.native.sync()
+            bb.free()
