@@ -161,7 +161,6 @@ typedef struct {
     const uint16_t *kc, *vc;
     const int32_t *pgtab;
     const cj_step_state *state;
-    int32_t *counters;       // per kv head arrival counters (merge in the last)
     int32_t n_q, n_kv, head_dim;
     int32_t splits;          // two-pass: the scores row stride (≥ count)
     int32_t pg_base;
@@ -170,8 +169,6 @@ typedef struct {
     int32_t workers;         // split-K: the CPU worker count the split rule uses
     float scale;
     int32_t pg_n;            // pages the sequence owns from pg_base (bounds the table prefetch)
-    int32_t per32;           // split-K with an output: pack `packed` at one scale per 32
-    uint8_t *packed;         // split-K with an output: the q8 pack of the merged output (may be null)
     // many-row forms (rowtab non-null): row r is sequence slot rowtab[2r] at
     // position states[slot].pos + rowtab[2r+1]; its pages from slot·pg_n
     const int32_t *rowtab;

@@ -14,9 +14,9 @@
 //   cpuDecodeSplits (:4879-4889) for a given worker count; one workgroup per
 //   (kv head, split slot); a split's positions run in order through an
 //   online softmax whose scores are the reference's 16 lane partials folded
-//   pairwise. cj_attn_merge (or, with an output, the last workgroup of a kv
-//   head) merges the splits as reducePackBlockCpu does (:5268-5400): four
-//   interleaved sub-sums.
+//   pairwise. cj_attn_merge (with a pack) or cj_attn_merge_q merges the
+//   splits as reducePackBlockCpu does (:5268-5400): four interleaved
+//   sub-sums.
 // cj_attn_scores_* + cj_attn_combine_*: attnScoreKernel (:397-425) and
 //   attnCombineKernel (:441-515): 32-lane strided dot + butterfly, then 128
 //   lanes for exp and sum (stride-halving tree) and the ascending-t sum of
@@ -61,8 +61,9 @@ DEV void attn_window(const cj_attn_args &a, int &count, int &from) {
 //            (the reference rescales only there) and the weight exp(s − m);
 //   update   lane d: acc·c (only where the maximum rose) then + v·w, in
 //            position order, each position's c and w read from its lane.
-// The last workgroup of a kv head to finish merges the head's splits and
-// writes the merged output and its q8 pack.
+// The merge is a launch of its own: in the last workgroup of each kv head it
+// waited for device-scope fences across the XCDs (2049 positions, 32/8 heads:
+// 48.9 us in one launch, 8.6 + 2.6 in two).
 template <int G>
 DEV void split_body(const cj_attn_args &a) {
     constexpr int HD = 128, TP = 64, KS = HD + 8, PGMAX = 256, HW = G / 4;
@@ -70,8 +71,6 @@ DEV void split_body(const cj_attn_args &a) {
     __shared__ __align__(16) uint16_t vs[TP][HD];
     __shared__ __align__(16) float qs[G][HD];
     __shared__ int pgs[PGMAX];
-    __shared__ float bmax[8];
-    __shared__ int ticket;
     __shared__ uint64_t etab[32];
     cj_exp_table(etab);   // visible after the tile loop's first barrier
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
@@ -190,59 +189,6 @@ DEV void split_body(const cj_attn_args &a) {
             if (lane == 0) *(float2 *)(pb + HD) = make_float2(m[hh], l[hh]);
         }
     }
-    if (!a.out && !a.packed) return;
-
-    // the last workgroup of this kv head merges its splits
-    __threadfence();
-    __syncthreads();
-    if (t == 0) ticket = atomicAdd(&a.counters[kvh], 1);
-    __syncthreads();
-    if (ticket != ATTN_MAX_SPLITS - 1) return;
-    __threadfence();
-    float *ob = (float *)&vs[0][0];                  // G·HD merged values (LDS reuse)
-#pragma unroll 1
-    for (int hh = 0; hh < HW; hh++) {
-        const int qq = kvh * G + wave + 4 * hh;
-        const float *pb0 = a.part + (int64_t)qq * ATTN_MAX_SPLITS * (HD + 2);
-        // lane s: split s's (max, sum); the weights of the merge
-        const float2 ml = *(const float2 *)(pb0 + lane * (HD + 2) + HD);
-        const bool in = lane < splits;
-        const float mv = in ? ml.x : -3.0e38f;
-        const float gm = group_max<64>(mv);
-        const bool on = in && ml.y > 0.0f;
-        const float wt = on ? cj_expf(mv - gm, etab) : 0.0f;
-        const uint64_t ons = __ballot(on);
-        float gl[4] = {0.0f, 0.0f, 0.0f, 0.0f}, ac0[4] = {0.0f, 0.0f, 0.0f, 0.0f}, ac1[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int s0 = 0; s0 < splits; s0 += 16) {
-            float2 av[16];
-#pragma unroll
-            for (int k = 0; k < 16; k++) av[k] = *(const float2 *)(pb0 + (s0 + k) * (HD + 2) + 2 * lane);
-#pragma unroll
-            for (int k = 0; k < 16; k++) {
-                const int s2 = s0 + k;
-                if (s2 < splits && ((ons >> s2) & 1)) {
-                    const float w = lane_f(wt, s2), lsv = lane_f(ml.y, s2);
-                    gl[k & 3] = __fadd_rn(gl[k & 3], __fmul_rn(w, lsv));
-                    ac0[k & 3] = __fadd_rn(ac0[k & 3], __fmul_rn(av[k].x, w));
-                    ac1[k & 3] = __fadd_rn(ac1[k & 3], __fmul_rn(av[k].y, w));
-                }
-            }
-        }
-        const float gt = __fadd_rn(__fadd_rn(__fadd_rn(gl[0], gl[1]), gl[2]), gl[3]);
-        const float rs = __fdiv_rn(1.0f, gt);
-        const float o0 = __fmul_rn(__fadd_rn(__fadd_rn(__fadd_rn(ac0[0], ac0[1]), ac0[2]), ac0[3]), rs);
-        const float o1 = __fmul_rn(__fadd_rn(__fadd_rn(__fadd_rn(ac1[0], ac1[1]), ac1[2]), ac1[3]), rs);
-        if (a.out) *(float2 *)(a.out + (int64_t)qq * HD + 2 * lane) = make_float2(o0, o1);
-        *(float2 *)(ob + (wave + 4 * hh) * HD + 2 * lane) = make_float2(o0, o1);
-    }
-    if (a.packed) {
-        __syncthreads();
-        // the kv head's G·HD outputs are G·HD/256 whole pack blocks
-#pragma unroll
-        for (int b = 0; b < G * HD / 256; b++)
-            pack256(ob[256 * b + t], a.per32, a.packed + ((int64_t)kvh * (G * HD / 256) + b) * 320, bmax);
-    }
-    if (t == 0) a.counters[kvh] = 0;
 }
 
 // The many-row form (batched decode): workgroup (row, kv head, split slot);

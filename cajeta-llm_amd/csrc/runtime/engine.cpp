@@ -109,7 +109,7 @@ struct Engine {
     float *hs_last = nullptr;  // the buffer the last enqueued step's residual ended in
     uint8_t *act_pack = nullptr, *attn_pack = nullptr, *xpack = nullptr;
     float *xn = nullptr;       // the normed residual as f32 (f32-activation consumers)
-    int32_t *glu_counters = nullptr, *argmax_counter = nullptr, *attn_counters = nullptr;
+    int32_t *glu_counters = nullptr, *argmax_counter = nullptr;
     float *part_v = nullptr;
     int32_t *part_i = nullptr;
     float *moe_logits = nullptr, *moe_w = nullptr, *moe_y = nullptr;
@@ -517,7 +517,6 @@ int Engine::load(const std::string &path, int ctx_, int max_seqs_, int kv_pages_
     part = (float *)alloc((size_t)n_heads * std::max<int64_t>(64 * (head_dim + 2), ctx) * 4);
     glu_counters = (int32_t *)alloc((size_t)fpad / 256 * 4 + 64);
     argmax_counter = (int32_t *)alloc(64);
-    attn_counters = (int32_t *)alloc((size_t)n_kv * 4 + 64);
     const int64_t max_wg = (vocab + 3) / 4 + 64;
     part_v = (float *)alloc((size_t)max_wg * 4);
     part_i = (int32_t *)alloc((size_t)max_wg * 4);
@@ -527,11 +526,10 @@ int Engine::load(const std::string &path, int ctx_, int max_seqs_, int kv_pages_
     route_status = (int32_t *)alloc(64);
     moe_y = (float *)alloc((size_t)hidden * std::max(1, n_used) * 4);
     if (!hs || !hs2 || !q || !attn || !act || !act_pack || !attn_pack || !xpack || !xn || !logits || !part || !glu_counters || !argmax_counter ||
-        !attn_counters || !part_v || !part_i || !moe_logits || !moe_w || !moe_sel || !moe_y || !route_status)
+        !part_v || !part_i || !moe_logits || !moe_w || !moe_sel || !moe_y || !route_status)
         return fail(CJ_ERR_HIP, "model: out of device memory (scratch)");
     CJ_HIP(hipMemset(glu_counters, 0, (size_t)fpad / 256 * 4 + 64));
     CJ_HIP(hipMemset(argmax_counter, 0, 64));
-    CJ_HIP(hipMemset(attn_counters, 0, (size_t)n_kv * 4 + 64));
     CJ_HIP(hipMemset(route_status, 0, 64));
 
     if (hipHostMalloc((void **)&pinned, (size_t)(ctx + 2) * 4 + sizeof(cj_step_state) + 64, 0) != hipSuccess)
@@ -692,7 +690,7 @@ int Engine::enqueue_step(int s) {
             probe(K_ATTN);
             cj_attn_args a{};
             a.part = part; a.out = attn; a.q = q; a.kc = L.kc; a.vc = L.vc; a.pgtab = pgtab; a.state = S.state;
-            a.counters = attn_counters; a.n_q = n_heads; a.n_kv = n_kv; a.head_dim = head_dim; a.workers = workers;
+            a.n_q = n_heads; a.n_kv = n_kv; a.head_dim = head_dim; a.workers = workers;
             a.pg_base = S.pg_base; a.pg_n = pages_per_seq; a.window = L.window; a.scale = scale;
             if (split) {
                 // partials, then the merge (a launch boundary orders them: a

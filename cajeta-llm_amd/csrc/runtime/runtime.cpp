@@ -878,12 +878,17 @@ int32_t cj_attend(int64_t part, int64_t out, int64_t q, int64_t kcache, int64_t 
     cj_attn_args a{};
     a.part = (float *)dptr(part); a.out = (float *)dptr(out); a.q = (const float *)dptr(q);
     a.kc = (const uint16_t *)dptr(kcache); a.vc = (const uint16_t *)dptr(vcache); a.pgtab = (const int32_t *)dptr(pgtab);
-    a.counters = (int32_t *)dptr(counters); a.n_q = n_q; a.n_kv = n_kv; a.head_dim = head_dim;
+    a.n_q = n_q; a.n_kv = n_kv; a.head_dim = head_dim;
     a.pg_base = pg_base; a.pg_n = (int32_t)pages; a.count = count; a.from = from; a.window = 0; a.workers = workers; a.scale = scale;
     char name[64];
     if (split) {
         snprintf(name, sizeof name, "cj_attn_split_h128_g%d", grp);
-        return launch(name, (uint32_t)(n_kv * 64), 256, 0, a);
+        const int32_t rc = launch(name, (uint32_t)(n_kv * 64), 256, 0, a);
+        if (rc || !out) return rc;
+        cj_merge_args m{};
+        m.out = a.out; m.part = a.part; m.n_q = n_q; m.head_dim = head_dim; m.n_kv = n_kv;
+        m.splits = cj_decode_splits(count, n_kv, workers);
+        return launch("cj_attn_merge_q", (uint32_t)(n_q * (head_dim / 32)), 128, 0, m);
     }
     a.splits = count;   // the scores row stride
     snprintf(name, sizeof name, "cj_attn_scores_h%d", head_dim);
