@@ -331,6 +331,34 @@ DEV void pack256(float v, int per32, uint8_t *ob, float *bmax) {
     lds_barrier();
 }
 
+// One 256-wide pack block by one wave, lane l holding elements 4l .. 4l+3:
+// pack256's values (maxima and integer sums do not depend on the order),
+// without LDS or barriers; eight lanes are a 32-group.
+DEV void pack_wave(const float (&v)[4], int per32, uint8_t *ob, int lane) {
+    float m = xmax8(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+    if (!per32) m = xmax64(m);
+    const float inv = m > 0.0f ? __fdiv_rn(127.0f, m) : 0.0f;
+    uint32_t w = 0u;
+    int s = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int q = round_away(__fmul_rn(v[k], inv));
+        s += q;
+        w |= ((uint32_t)q & 255u) << (8 * k);
+    }
+    *(uint32_t *)(ob + 4 * lane) = w;
+    s += dpp_i<DPP_XOR1>(s);
+    s += dpp_i<DPP_XOR2>(s);
+    s += dpp_i<DPP_HMIRROR>(s);
+    if ((lane & 7) == 0) *(int32_t *)(ob + 256 + 4 * (lane >> 3)) = s;
+    if (per32) {
+        if ((lane & 7) == 0) *(float *)(ob + 288 + 4 * (lane >> 3)) = __fdiv_rn(m, 127.0f);
+    } else {
+        if (lane == 0) *(float *)(ob + 288) = __fdiv_rn(m, 127.0f);
+        pack_zero_pad(ob, lane);
+    }
+}
+
 // Lane-uniform reads of another lane's value (the lane index must be the
 // same on every lane of the wave).
 DEV float lane_f(float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }

@@ -25,6 +25,30 @@ extern "C" __global__ void __launch_bounds__(256) cj_pack(cj_pack_args a) {
     for (int i = threadIdx.x; i < nblk * 20; i += 256) ((uint4 *)o)[i] = ((const uint4 *)sx)[i];
 }
 
+// The pack alone, a wave a 256-wide block (four a workgroup, over all the
+// rows' blocks). Bound by latency at one row: a workgroup a row, as cj_pack,
+// walked a 14336-wide row's 56 blocks on one CU (with the Q4_K product after
+// it, 12.4 us a pass; 10.0 with this).
+extern "C" __global__ void __launch_bounds__(256) cj_pack_blocks(cj_pack_args a) {
+    const int lane = threadIdx.x & 63;
+    const int64_t nblk = a.npad / 256, i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (i >= nblk * a.rows) return;
+    const int64_t row = i / nblk, blk = i % nblk, e = blk * 256 + 4 * lane;
+    const float *x = a.x + row * a.n;
+    float v[4];
+    if (a.n % 4 == 0 && ((uintptr_t)a.x & 15) == 0) {   // every group of four whole and aligned
+        const float4 q = e < a.n ? *(const float4 *)(x + e) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const float q = x[min(e + k, a.n - 1)];
+            v[k] = e + k < a.n ? q : 0.0f;
+        }
+    }
+    pack_wave(v, a.per32, a.out + i * 320, lane);
+}
+
 // RMSNorm + pack of one row, one workgroup per 256-wide block. Every
 // workgroup forms the row's sum of squares itself in the reference order
 // (thread t: x[t + 256k], k ascending, ragged past the width, then the

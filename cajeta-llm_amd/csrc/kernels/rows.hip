@@ -96,36 +96,7 @@ extern "C" __global__ void __launch_bounds__(256) cj_rows_glu(cj_rows_args a) {
 #pragma unroll
         for (int k = 0; k < 4; k++) if (e0 + k < a.n) o[e0 + k] = v[k];
     }
-    float m = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-    m = fmaxf(m, __shfl_xor(m, 1));
-    m = fmaxf(m, __shfl_xor(m, 2));
-    m = fmaxf(m, __shfl_xor(m, 4));    // the 32-group (eight lanes)
-    if (!a.per32) {
-        m = fmaxf(m, __shfl_xor(m, 8));
-        m = fmaxf(m, __shfl_xor(m, 16));
-        m = fmaxf(m, __shfl_xor(m, 32));
-    }
-    const float inv = m > 0.0f ? __fdiv_rn(127.0f, m) : 0.0f;
-    uint32_t w = 0u;
-    int s = 0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const int q = round_away(__fmul_rn(v[k], inv));
-        s += q;
-        w |= ((uint32_t)q & 255u) << (8 * k);
-    }
-    uint8_t *ob = a.packed + (int64_t)r * a.pack_stride + blk * 320;
-    *(uint32_t *)(ob + 4 * lane) = w;
-    s += __shfl_xor(s, 1);
-    s += __shfl_xor(s, 2);
-    s += __shfl_xor(s, 4);
-    if ((lane & 7) == 0) *(int32_t *)(ob + 256 + 4 * (lane >> 3)) = s;
-    if (a.per32) {
-        if ((lane & 7) == 0) *(float *)(ob + 288 + 4 * (lane >> 3)) = __fdiv_rn(m, 127.0f);
-    } else {
-        if (lane == 0) *(float *)(ob + 288) = __fdiv_rn(m, 127.0f);
-        pack_zero_pad(ob, lane);
-    }
+    pack_wave(v, a.per32, a.packed + (int64_t)r * a.pack_stride + blk * 320, lane);
 }
 
 // First-occurrence argmax partials: chunk c (1024 wide) of row r's logits →

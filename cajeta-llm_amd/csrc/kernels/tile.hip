@@ -474,3 +474,166 @@ extern "C" __global__ void __launch_bounds__(512) cj_gemm_t_q6k(cj_gemv_args a) 
     }
     mt_write(a, r0 + 32 * wr + m, c0 + 32 * wc + 4 * hf, acc);
 }
+
+// ------------------------------------------------------------------- Q8_0
+
+// The same copies into LDS: a group of 8 blocks is 256 code bytes a row and
+// a column, word w of either at w ^ (row or column % 16). Per output and
+// block the reference's rounded steps are fs = Σ_j (d_j·xs_j)·dot_j over the
+// group's blocks, then acc += fs; the d·xs of two blocks are one outer
+// product (v_mfma_f32_32x32x1_2b_f32, one rounding a product, checked on the
+// part against the f32 multiply with denormals). A short last group repeats
+// the row's last block under scales of zero, whose terms (±0) change no sum.
+typedef float f32x32 __attribute__((ext_vector_type(32)));
+
+#define M8_A 0                                        // [64 rows][256]
+#define M8_B (MT_ROWS * 256)                          // [128 columns][256]
+#define M8_BUF (M8_B + MT_COLS * 256)
+#define M8_T (2 * M8_BUF)                             // two groups' scales:
+#define M8_D 0                                        //   f32 [8][64 rows]
+#define M8_XS (8 * MT_ROWS * 4)                       //   f32 [8][128 columns]
+#define M8_TAB (M8_XS + 8 * MT_COLS * 4)
+#define M8_LDS (M8_T + 2 * M8_TAB)
+
+// fl(a·b) for a of lane l % 32 as D's row and b of lane l % 32 as its column;
+// lanes 0..31 give the first 16 results' operands, 32..63 the others'
+DEV f32x32 mt_outer(float a, float b) {
+    f32x32 z;
+#pragma unroll
+    for (int i = 0; i < 32; i++) z[i] = 0.0f;
+    return __builtin_amdgcn_mfma_f32_32x32x1f32(a, b, z, 0, 0, 0);
+}
+
+// Blocks 2p and 2p + 1 of a group: their integer dots and scale products.
+struct M8Pair {
+    i32x16 d0, d1;
+    f32x32 s;
+    // ao, bo: the lane's row and column in the buffer, its swizzle in bits 4..7
+    DEV void dot(const uint8_t *buf, const uint8_t *T, int ao, int bo, int p, int row, int col, int hf, const i32x16 &M) {
+        d0 = mt_dot(*(const i32x4 *)(buf + (bo ^ (64 * p))), *(const i32x4 *)(buf + (ao ^ (64 * p))), M);
+        d1 = mt_dot(*(const i32x4 *)(buf + (bo ^ (64 * p + 32))), *(const i32x4 *)(buf + (ao ^ (64 * p + 32))), M);
+        s = mt_outer(*(const float *)(T + M8_XS + ((2 * p + hf) * MT_COLS + col) * 4),
+                     *(const float *)(T + M8_D + ((2 * p + hf) * MT_ROWS + row) * 4));
+    }
+    template <bool FIRST>
+    DEV void fold(f32x16 &fs) const {
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const float t0 = __fmul_rn(s[i], mt_sum(d0[i]));
+            fs[i] = FIRST ? t0 : __fadd_rn(fs[i], t0);
+            fs[i] = __fadd_rn(fs[i], __fmul_rn(s[16 + i], mt_sum(d1[i])));
+        }
+    }
+};
+
+struct M8 {
+    const uint8_t *asrc[2], *bsrc[4], *ssrc;
+    uint8_t *lds;
+    int64_t nb32;
+    int t, wave, row, col, hf, ng, word;
+    u32x4 e;
+    f32x16 acc;
+
+    DEV void init(const cj_gemv_args &a, uint8_t *l, int64_t r0, int64_t c0) {
+        lds = l;
+        t = threadIdx.x;
+        wave = __builtin_amdgcn_readfirstlane(t >> 6);
+        hf = (t >> 5) & 1;
+        row = 32 * (wave >> 2) + (t & 31);
+        col = 32 * (wave & 3) + (t & 31);
+        nb32 = a.cols / 32;
+        ng = (int)((a.cols + 255) / 256);
+        const int lane = t & 63;
+        // rows 8·wave + 4·i + lane / 16, columns 16·wave + 4·i + lane / 16
+#pragma unroll
+        for (int i = 0; i < 2; i++) asrc[i] = a.w + min(r0 + 8 * wave + 4 * i + (lane >> 4), a.rows - 1) * a.row_bytes;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int c = 16 * wave + 4 * i + (lane >> 4);
+            bsrc[i] = a.xp + min(c0 + c, (int64_t)a.batch - 1) * a.xp_stride + 16 * ((lane & 15) ^ (c & 15));
+        }
+        // threads 0..255: four of a column's scales; 256..319: a row's eight
+        if (t < 256) ssrc = a.xp + min(c0 + (t >> 1), (int64_t)a.batch - 1) * a.xp_stride + 288 + 16 * (t & 1);
+        else ssrc = a.w + min(r0 + (t & 63), a.rows - 1) * a.row_bytes + nb32 * 32;
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[i] = 0.0f;
+    }
+    DEV void copy(int g, int buf) {
+        const int lane = t & 63;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int w = (lane & 15) ^ ((8 * wave + 4 * i + (lane >> 4)) & 15);
+            const int64_t blk = min((int64_t)8 * g + (w >> 1), nb32 - 1);
+            mt_dma(asrc[i] + blk * 32 + 16 * (w & 1), lds + buf * M8_BUF + M8_A + wave * 2048 + i * 1024);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) mt_dma(bsrc[i] + (int64_t)g * 320, lds + buf * M8_BUF + M8_B + wave * 4096 + i * 1024);
+    }
+    DEV void fetch(int g) {
+        if (t < 256) e = *(const u32x4 *)(ssrc + (int64_t)g * 320);
+        else if (wave == 4) e = *(const u32x4 *)(ssrc + (int64_t)g * 16);
+    }
+    DEV void table(int g, int buf) {
+        uint8_t *T = lds + M8_T + buf * M8_TAB;
+        const int nj = (int)min(nb32 - 8 * (int64_t)g, (int64_t)8);
+        if (t < 256) {
+            const int c = t >> 1, j0 = 4 * (t & 1);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                *(float *)(T + M8_XS + ((j0 + j) * MT_COLS + c) * 4) = j0 + j < nj ? __uint_as_float(e[j]) : 0.0f;
+        } else if (wave == 4) {
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                *(float *)(T + M8_D + (j * MT_ROWS + (t & 63)) * 4) = j < nj ? h2f(e[j >> 1] >> (16 * (j & 1))) : 0.0f;
+        }
+    }
+    // One pair's products are formed while the pair before is folded. The
+    // empty asm ties a pair's operand addresses to the fold two before it:
+    // left free, the compiler issues all the products first and spills their
+    // results.
+    DEV void group(int buf) {
+        const uint8_t *b = lds + buf * M8_BUF, *T = lds + M8_T + buf * M8_TAB;
+        const i32x16 M = mt_magic();
+        int ao = M8_A + row * 256 + 16 * ((row & 15) ^ hf), bo = M8_B + col * 256 + 16 * ((col & 15) ^ hf);
+        f32x16 fs;
+        M8Pair P, Q;
+        P.dot(b, T, ao, bo, 0, row, col, hf, M);
+        Q.dot(b, T, ao, bo, 1, row, col, hf, M);
+        P.fold<true>(fs);
+        asm volatile("" : "+v"(ao), "+v"(bo), "+v"(fs));
+        P.dot(b, T, ao, bo, 2, row, col, hf, M);
+        Q.fold<false>(fs);
+        asm volatile("" : "+v"(ao), "+v"(bo), "+v"(fs));
+        Q.dot(b, T, ao, bo, 3, row, col, hf, M);
+        P.fold<false>(fs);
+        Q.fold<false>(fs);
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[i] = __fadd_rn(acc[i], fs[i]);
+    }
+    DEV void step(int g, int buf) {
+        const int n = min(g + 1, ng - 1);
+        copy(n, buf ^ 1);
+        group(buf);
+        table(n, buf ^ 1);
+        mt_sync();
+        fetch(min(g + 2, ng - 1));
+    }
+};
+
+extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) cj_gemm_t_q80(cj_gemv_args a) {
+    __shared__ __align__(16) uint8_t mt_lds[M8_LDS];
+    int64_t r0, c0;
+    if (!mt_tile(a, r0, c0)) return;
+    M8 W;
+    W.init(a, mt_lds, r0, c0);
+    W.fetch(0);
+    W.copy(0, 0);
+    W.table(0, 0);
+    mt_sync();
+    W.fetch(min(1, W.ng - 1));
+    for (int g = 0; g < W.ng; g += 2) {
+        W.step(g, 0);
+        if (g + 1 < W.ng) W.step(g + 1, 1);
+    }
+    mt_write(a, r0 + W.row, c0 + 32 * (W.wave & 3) + 4 * W.hf, W.acc);
+}

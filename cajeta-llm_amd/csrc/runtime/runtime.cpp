@@ -374,13 +374,16 @@ bool gemm_supported(int type) { return type == CJ_Q8_0 || type == CJ_Q4_K || typ
 //    other kernel's 30 us (2048 × 128: 29.6 → 32.7 stays; 6144 × 64: 42.5 →
 //    32.4; 28672 × 17: 81 → 64; 4096 × 512: 209 → 35.5).
 static bool gemm_tiled(const cj_gemv_args &a, int64_t &wgs) {
-    if ((a.type != CJ_Q4_K && a.type != CJ_Q6_K) || a.batch <= 16) return false;
+    if (a.batch <= 16) return false;
+    static const char *t8 = getenv("CJ_T8");
+    if (a.type == CJ_Q8_0 && !t8) return false;
     // its copies into LDS move aligned 16-byte words
     if ((((uintptr_t)a.w | (uintptr_t)a.xp | (uintptr_t)a.xp_stride | (uintptr_t)a.row_bytes) & 15) != 0) return false;
     const int64_t cus = std::max(1, g.cus), gx = ((int64_t)a.batch + 127) / 128, gy = (a.rows + 63) / 64;
     const int64_t rounds = (gx * gy + cus - 1) / cus;
     wgs = gx * (gy >= 8 ? (gy + 7) / 8 * 8 : gy);
     if (wgs > 0x7fffffff || (a.type == CJ_Q4_K && gy > 65535)) return false;
+    if (a.type == CJ_Q8_0) return atoi(t8) > 0;
     if (a.type == CJ_Q4_K) return gy * (((int64_t)a.batch + 31) / 32) > cus * rounds;
     return a.rows * (((int64_t)a.batch + 15) / 16 * 16) > 1200 * cus * rounds;
 }
@@ -410,8 +413,8 @@ int run_gemm(const cj_gemv_args &a) {
     }
     int64_t wgs = 0;
     if (gemm_tiled(a, wgs)) {
-        if (a.cols % 256) return fail(CJ_ERR_ARG, "gemm: K-quant rows are whole 256-element blocks");
-        return launch(a.type == CJ_Q4_K ? "cj_gemm_t_q4k" : "cj_gemm_t_q6k", (uint32_t)wgs, 512, 0, a);
+        if (a.type != CJ_Q8_0 && a.cols % 256) return fail(CJ_ERR_ARG, "gemm: K-quant rows are whole 256-element blocks");
+        return launch(a.type == CJ_Q8_0 ? "cj_gemm_t_q80" : a.type == CJ_Q4_K ? "cj_gemm_t_q4k" : "cj_gemm_t_q6k", (uint32_t)wgs, 512, 0, a);
     }
     if (a.type == CJ_Q6_K) {
         // many-column GEMV (4 or 8 columns a grid row; its LDS fixed: a
@@ -482,12 +485,12 @@ int32_t cj_init(int32_t device) {
         "cj_gemv_q40b_r2", "cj_gemv_q40b_r4", "cj_gemm_q40_r2_c4", "cj_gemm_q40_r4_c4",
         "cj_gemv_mxfp4", "cj_gemv_f32", "cj_gemv_mxfp4_r32", "cj_gemv_f32_r32", "cj_gemv_mxfp4_r1", "cj_gemv_f32_r1",
         "cj_moe_combine", "cj_moe_combine_norm",
-        "cj_pack", "cj_norm_pack", "cj_norm_pack_rows", "cj_copy", "cj_page_span", "cj_glu", "cj_add", "cj_dequant", "cj_prepare", "cj_embed", "cj_argmax",
+        "cj_pack", "cj_pack_blocks", "cj_norm_pack", "cj_norm_pack_rows", "cj_copy", "cj_page_span", "cj_glu", "cj_add", "cj_dequant", "cj_prepare", "cj_embed", "cj_argmax",
         "cj_attn_split_h128_g4", "cj_attn_split_h128_g8", "cj_attn_scores_h64", "cj_attn_scores_h128",
         "cj_attn_combine_h64", "cj_attn_combine_h128", "cj_attn_fused_h64", "cj_attn_fused_h128",
         "cj_attn_merge", "cj_attn_merge_q", "cj_moe_group", "cj_argmax_pick", "cj_qkprep", "cj_zero", "cj_moe_route", "cj_router_topk",
         "cj_gemm_q80_n2", "cj_gemm_q4k_n2", "cj_gemm_q80_n4", "cj_gemm_q6k_c4", "cj_gemm_q6k_c8", "cj_gemm_q6k_m16",
-        "cj_gemm_sk_q80_n1", "cj_gemm_sk_q80_n2", "cj_gemm_sk_q4k_n1", "cj_gemm_t_q4k", "cj_gemm_t_q6k",
+        "cj_gemm_sk_q80_n1", "cj_gemm_sk_q80_n2", "cj_gemm_sk_q4k_n1", "cj_gemm_t_q4k", "cj_gemm_t_q6k", "cj_gemm_t_q80",
         "cj_rows_embed", "cj_rows_qkv", "cj_rows_glu", "cj_rows_argmax", "cj_rows_pick",
         "cj_attn_split_rows_h128_g4", "cj_attn_split_rows_h128_g8", "cj_attn_merge_rows",
         "cj_attn_prefill_h128_g1", "cj_attn_prefill_h128_g2", "cj_attn_prefill_h128_g4", "cj_attn_prefill_h128_g8",
@@ -691,7 +694,9 @@ int32_t cj_q8k_pack(int64_t out, int64_t x, int64_t rows, int64_t n, int64_t npa
         return fail(CJ_ERR_ARG, "cj_q8k_pack: buffers smaller than %lld rows", (long long)rows);
     cj_pack_args a{};
     a.out = (uint8_t *)dptr(out); a.x = (const float *)dptr(x); a.n = n; a.npad = npad; a.rows = rows; a.per32 = per32;
-    return launch("cj_pack", (uint32_t)rows, 256, (uint32_t)(npad / 256 * 320), a);
+    const int64_t wgs = (npad / 256 * rows + 3) / 4;
+    if (wgs > 0x7fffffff) return launch("cj_pack", (uint32_t)rows, 256, (uint32_t)(npad / 256 * 320), a);
+    return launch("cj_pack_blocks", (uint32_t)wgs, 256, 0, a);
 }
 
 int32_t cj_rmsnorm_pack(int64_t out, int64_t packed, int64_t x, int64_t w, int64_t dim, float eps, int32_t form, int32_t per32) {

@@ -754,3 +754,21 @@ def test_page_table_checks(gpu, O, pages):
             assert attend() == 0
             gpu.native.sync()
             bb.free()
+
+
+@pytest.mark.parametrize("per32", [0, 1])
+@pytest.mark.parametrize("rows,n,off", [(1, 14336, 0), (3, 2880, 0), (5, 1408, 1), (7, 32, 0), (2, 777, 3), (513, 256, 0)])
+def test_pack_rows_of_any_width(gpu, O, per32, rows, n, off):
+    """cj_q8k_pack over several rows: widths that are not whole blocks or
+    fours, rows off the 16-byte lines, and a last workgroup that is not full."""
+    say("pack rows", per32, rows, n, off)
+    rng = np.random.default_rng(rows * n + per32)
+    npad = (n + 255) // 256 * 256
+    x = rng.standard_normal(off + rows * n).astype(np.float32)
+    x[off:off + min(n, 32)] = 0.0
+    xb, ob = gpu.Buffer.of(x), gpu.Buffer(rows * npad // 256 * 320)
+    gpu.native.check(gpu.native.lib().cj_q8k_pack(ob.h, xb.h + 4 * off, rows, n, npad, per32), "pack")
+    got = ob.download(np.uint8, rows * npad // 256 * 320).reshape(rows, -1)
+    for r in range(rows):
+        ref = O.q8k_pack(x[off + r * n:off + (r + 1) * n], per32=bool(per32), npad=npad)
+        assert np.array_equal(got[r], ref), "row %d" % r
