@@ -34,10 +34,12 @@
 // D[8·(i / 4) + 4·(l / 32) + i % 4][l % 32], i < 16. The activations are the
 // first operand, so a lane's 16 results are 16 columns of one weight row.
 //
-// Measured (MI355X, 512 columns, us): Q4_K 4096×14336 253 → 104, 14336×4096
-// → 127; Q6_K 4096×14336 at 203 columns 283 → 89; what is left above the
-// VALU's issue time is the step's barrier and the issue of its copies, with
-// two waves a SIMD to cover them.
+// Measured (MI355X, 512 columns, us): Q4_K 4096×14336 253 → 102, 28672×4096
+// 233; Q8_0 14336×4096 169 → 131.5, 4096×4096 52 → 33; Q6_K 4096×14336 at
+// 203 columns 283 → 89. A step (Q4_K, cycles, clock stamps of a wave): the
+// sub-blocks' products and folds 1,800–2,100 — the two waves' VALU issue
+// time — the block's fold 650, the table 200; the rest is the barrier and
+// the copies' issue, which two waves a SIMD do not cover.
 #include "common.h"
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -161,10 +163,7 @@ struct MnQ4 {
         const int pc = 2 * k + (wave >> 2);
         mt_dma(asrc + (pc * nb + min(4 * s + ablk, nb - 1)) * 16, lds + MN_A + (s & 1) * 32768 + pc * 4096 + (wave & 3) * 1024);
     }
-    DEV void copy_b(int64_t b, int buf) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) mt_dma(bsrc[i] + b * 320, lds + MN_B + buf * 32768 + wave * 4096 + i * 1024);
-    }
+    DEV void copy_b(int64_t b, int buf, int i) { mt_dma(bsrc[i] + b * 320, lds + MN_B + buf * 32768 + wave * 4096 + i * 1024); }
     DEV void fetch(int64_t b) {
         if (t < 256) {
             e = *(const u32x4 *)(esrc + b * 320 + 16 * (t & 1));
@@ -214,9 +213,9 @@ struct MnQ4 {
             *(float *)(T + MN_D + (MT_ROWS + r) * 4) = h2f(e.x >> 16);
         }
     }
-    // block K of superblock s
-    template <int K>
-    DEV void block(int64_t s) {
+    // block K of superblock s; mid(j) runs after sub-block j's fold
+    template <int K, class Mid>
+    DEV void block(int64_t s, Mid &&mid) {
         const int row = 32 * wr + m, col = 32 * wc + m;
         const uint8_t *ap = lds + MN_A + (s & 1) * 32768 + hf * 4096 + row * 64 + 16 * (K ^ ((row >> 2) & 3));
         const uint8_t *T = lds + MN_T + (K & 1) * MN_TAB;
@@ -255,6 +254,7 @@ struct MnQ4 {
             // the product after next waits for this fold (left free, the
             // compiler issues all eight first and spills their results)
             if (j < 6) asm volatile("" : "+v"(x[j + 2]), "+v"(S));
+            mid(j);
         }
         f32x16 Dm;
 #pragma unroll
@@ -276,9 +276,18 @@ struct MnQ4 {
     DEV bool step(int64_t s) {
         const int64_t b = 4 * s + K;
         if (b >= nb) return true;
-        copy_b(min(b + 1, nb - 1), (K + 1) & 1);
-        copy_a(s + 1, K);
-        block<K>(s);
+        const int64_t n = min(b + 1, nb - 1);
+        // the copies spread over the first sub-blocks: issued together, the
+        // waves queue on the address unit (Q8_0 14336×4096 × 512: 138 → 131.5 us,
+        // Q4_K 4096×14336 × 512: 104.6 → 102.2; spread to the step's end they
+        // come late: 152, 113)
+        block<K>(s, [&](int j) {
+            if (j < 2) {
+                copy_b(n, (K + 1) & 1, 2 * j);
+                copy_b(n, (K + 1) & 1, 2 * j + 1);
+            }
+            if (j == 2) copy_a(s + 1, K);
+        });
         table((K + 1) & 1);
         mt_sync();
         fetch(min(b + 2, nb - 1));
@@ -295,7 +304,8 @@ extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_pe
     W.fetch(0);
 #pragma unroll
     for (int k = 0; k < 4; k++) W.copy_a(0, k);
-    W.copy_b(0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; i++) W.copy_b(0, 0, i);
     W.table(0);
     mt_sync();
     W.fetch(min((int64_t)1, W.nb - 1));
@@ -558,17 +568,12 @@ struct M8 {
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[i] = 0.0f;
     }
-    DEV void copy(int g, int buf) {
-        const int lane = t & 63;
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int w = (lane & 15) ^ ((8 * wave + 4 * i + (lane >> 4)) & 15);
-            const int64_t blk = min((int64_t)8 * g + (w >> 1), nb32 - 1);
-            mt_dma(asrc[i] + blk * 32 + 16 * (w & 1), lds + buf * M8_BUF + M8_A + wave * 2048 + i * 1024);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) mt_dma(bsrc[i] + (int64_t)g * 320, lds + buf * M8_BUF + M8_B + wave * 4096 + i * 1024);
+    DEV void copy_a(int g, int buf, int i) {
+        const int lane = t & 63, w = (lane & 15) ^ ((8 * wave + 4 * i + (lane >> 4)) & 15);
+        const int64_t blk = min((int64_t)8 * g + (w >> 1), nb32 - 1);
+        mt_dma(asrc[i] + blk * 32 + 16 * (w & 1), lds + buf * M8_BUF + M8_A + wave * 2048 + i * 1024);
     }
+    DEV void copy_b(int g, int buf, int i) { mt_dma(bsrc[i] + (int64_t)g * 320, lds + buf * M8_BUF + M8_B + wave * 4096 + i * 1024); }
     DEV void fetch(int g) {
         if (t < 256) e = *(const u32x4 *)(ssrc + (int64_t)g * 320);
         else if (wave == 4) e = *(const u32x4 *)(ssrc + (int64_t)g * 16);
@@ -591,7 +596,8 @@ struct M8 {
     // empty asm ties a pair's operand addresses to the fold two before it:
     // left free, the compiler issues all the products first and spills their
     // results.
-    DEV void group(int buf) {
+    template <class Mid>
+    DEV void group(int buf, Mid &&mid) {
         const uint8_t *b = lds + buf * M8_BUF, *T = lds + M8_T + buf * M8_TAB;
         const i32x16 M = mt_magic();
         int ao = M8_A + row * 256 + 16 * ((row & 15) ^ hf), bo = M8_B + col * 256 + 16 * ((col & 15) ^ hf);
@@ -599,12 +605,15 @@ struct M8 {
         M8Pair P, Q;
         P.dot(b, T, ao, bo, 0, row, col, hf, M);
         Q.dot(b, T, ao, bo, 1, row, col, hf, M);
+        mid(0);
         P.fold<true>(fs);
         asm volatile("" : "+v"(ao), "+v"(bo), "+v"(fs));
         P.dot(b, T, ao, bo, 2, row, col, hf, M);
+        mid(1);
         Q.fold<false>(fs);
         asm volatile("" : "+v"(ao), "+v"(bo), "+v"(fs));
         Q.dot(b, T, ao, bo, 3, row, col, hf, M);
+        mid(2);
         P.fold<false>(fs);
         Q.fold<false>(fs);
 #pragma unroll
@@ -612,8 +621,13 @@ struct M8 {
     }
     DEV void step(int g, int buf) {
         const int n = min(g + 1, ng - 1);
-        copy(n, buf ^ 1);
-        group(buf);
+        group(buf, [&](int p) {   // (the copies spread over the step's start)
+            if (p < 2) {
+                copy_a(n, buf ^ 1, p);
+                copy_b(n, buf ^ 1, 2 * p);
+                copy_b(n, buf ^ 1, 2 * p + 1);
+            }
+        });
         table(n, buf ^ 1);
         mt_sync();
         fetch(min(g + 2, ng - 1));
@@ -627,7 +641,10 @@ extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_pe
     M8 W;
     W.init(a, mt_lds, r0, c0);
     W.fetch(0);
-    W.copy(0, 0);
+#pragma unroll
+    for (int i = 0; i < 2; i++) W.copy_a(0, 0, i);
+#pragma unroll
+    for (int i = 0; i < 4; i++) W.copy_b(0, 0, i);
     W.table(0, 0);
     mt_sync();
     W.fetch(min(1, W.ng - 1));

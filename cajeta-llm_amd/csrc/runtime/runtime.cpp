@@ -362,9 +362,9 @@ GemvPlan plan_gemv(int type, int64_t rows, int64_t cols, int target, int pro, in
 
 bool gemm_supported(int type) { return type == CJ_Q8_0 || type == CJ_Q4_K || type == CJ_Q6_K; }
 
-// The K-quants' 64-row × 128-column tile kernel (tile.hip) takes about
-// 2.05 us a 256-element block and round of tiles over the CUs, however full
-// the tiles are. Its lines, measured on 256 CUs (us, 4096 columns of weights
+// The 64-row × 128-column tile kernels (tile.hip) take about 2.05 us a
+// 256-element block and round of tiles over the CUs, however full the tiles
+// are. Their lines, measured on 256 CUs (us, 4096 columns of weights
 // unless named; other kernel → tile kernel):
 //  - Q4_K: where the 64 × 32 tiles of the other kernel are more than one a CU
 //    for each round (4096 × 128: 31.5 → 34.2 stays; 6144 × 96: 43.9 → 33.3;
@@ -372,18 +372,25 @@ bool gemm_supported(int type) { return type == CJ_Q8_0 || type == CJ_Q4_K || typ
 //    × 33: 84.2 → 66.8);
 //  - Q6_K: where rows × columns (in 16s) pass 1200 a CU for each round, the
 //    other kernel's 30 us (2048 × 128: 29.6 → 32.7 stays; 6144 × 64: 42.5 →
-//    32.4; 28672 × 17: 81 → 64; 4096 × 512: 209 → 35.5).
+//    32.4; 28672 × 17: 81 → 64; 4096 × 512: 209 → 35.5);
+//  - Q8_0, above 32 columns: against the split-K kernel where rows × columns
+//    (in 32s) pass 2200 a CU for each round (4096 × 64: 15.6 → 34 stays;
+//    14336 × 33: 48 → 34.5); against the 64 × 64 tiles in one round always
+//    (4096 × 512: 52 → 33; 14336 × 128: 51 → 36), in more where those tiles
+//    pass 1.37 a CU for each round (14336 × 512, four rounds: 169 → 131.5).
 static bool gemm_tiled(const cj_gemv_args &a, int64_t &wgs) {
-    if (a.batch <= 16) return false;
-    static const char *t8 = getenv("CJ_T8");
-    if (a.type == CJ_Q8_0 && !t8) return false;
+    if ((a.type != CJ_Q4_K && a.type != CJ_Q6_K && a.type != CJ_Q8_0) || a.batch <= (a.type == CJ_Q8_0 ? 32 : 16)) return false;
     // its copies into LDS move aligned 16-byte words
     if ((((uintptr_t)a.w | (uintptr_t)a.xp | (uintptr_t)a.xp_stride | (uintptr_t)a.row_bytes) & 15) != 0) return false;
     const int64_t cus = std::max(1, g.cus), gx = ((int64_t)a.batch + 127) / 128, gy = (a.rows + 63) / 64;
     const int64_t rounds = (gx * gy + cus - 1) / cus;
     wgs = gx * (gy >= 8 ? (gy + 7) / 8 * 8 : gy);
-    if (wgs > 0x7fffffff || (a.type == CJ_Q4_K && gy > 65535)) return false;
-    if (a.type == CJ_Q8_0) return atoi(t8) > 0;
+    if (wgs > 0x7fffffff || (a.type != CJ_Q6_K && gy > 65535)) return false;
+    if (a.type == CJ_Q8_0) {
+        const int64_t t64 = gy * (((int64_t)a.batch + 63) / 64);   // the other kernel's tiles
+        if (t64 < 256 && a.batch <= 64) return a.rows * (((int64_t)a.batch + 31) / 32 * 32) > 2200 * cus * rounds;
+        return rounds == 1 || 8 * t64 > 11 * cus * rounds;
+    }
     if (a.type == CJ_Q4_K) return gy * (((int64_t)a.batch + 31) / 32) > cus * rounds;
     return a.rows * (((int64_t)a.batch + 15) / 16 * 16) > 1200 * cus * rounds;
 }

@@ -678,21 +678,27 @@ def test_allocating_argmax_refuses_a_graph_capture(gpu):
     assert tb.download(np.int32, 1)[0] == 4999
 
 
-@pytest.mark.parametrize("name,ty", [("q4_k", 12), ("q6_k", 14)])
+@pytest.mark.parametrize("name,ty", [("q4_k", 12), ("q6_k", 14), ("q8_0", 8)])
 @pytest.mark.parametrize("rows,cols,ncols", [(4160, 256, 130), (4161, 1280, 129), (8200, 512, 127), (2050, 2304, 300),
-                                             (40, 768, 30000), (16448, 1024, 33)])
+                                             (40, 768, 30000), (16448, 1024, 33), (4160, 1312, 130),
+                                             (1030, 32, 300)])
 def test_matmul_tile_kernels(gpu, O, name, ty, rows, cols, ncols):
     """Shapes that take the 64-row × 128-column tile kernels (more tiles than
-    a CU's worth of the others'), off the tile's edges, one block to nine:
+    a CU's worth of the others'), off the tile's edges, one block to nine, and
+    for Q8_0 rows that end inside a 256-element group:
     every column checked bit for bit against the oracle's one-column product.
     Row 0 and column 0 hold the largest codes and scales, so their integer
     sums reach their bounds."""
+    if cols % 256 and ty != O.Q8_0:
+        pytest.skip("K-quant rows are whole 256-element blocks")
     say("matmul tile", name, rows, cols, ncols)
     rng = np.random.default_rng(rows + cols * 3 + ncols + ty)
     be, bb = O.BLOCK[ty]
     raw = rand_blocks(O, ty, rows * cols // be, rng).reshape(rows, cols // be, bb).copy()
     if ty == O.Q4_K:
         raw[0, :, 4:] = 0xFF                       # every scale, min and code at its largest
+    elif ty == O.Q8_0:
+        raw[0, :, 2:] = 0x80                       # every code −128
     else:
         raw[0, :, :192] = 0                        # every code −32
         raw[0, :, 192:208] = 0x80                  # every scale −128
@@ -703,10 +709,12 @@ def test_matmul_tile_kernels(gpu, O, name, ty, rows, cols, ncols):
     distinct = min(ncols, 40)                      # later columns repeat them
     x = rng.standard_normal((distinct, cols)).astype(np.float32)
     x[0] = 1.0
-    stride = cols // 256 * 320 + 32
+    stride = (cols + 255) // 256 * 320 + 32
     packs = np.zeros((ncols, stride), np.uint8)
     for c in range(distinct):
-        packs[c, :stride - 32] = O.q8k_pack(x[c])
+        packs[c, :stride - 32] = O.q8k_pack(x[c], per32=(ty == O.Q8_0), npad=(cols + 255) // 256 * 256)
+        if ty == O.Q8_0 and cols % 256:            # whatever stands past the row's blocks takes no part
+            packs[c, stride - 32 - 4 * (8 - cols % 256 // 32):stride - 32] = 0xFF
     packs[:] = packs[np.arange(ncols) % distinct]
     refs = np.stack([O.matvec_packed(ty, raw.reshape(-1), rows, cols, packs[c, :stride - 32]) for c in range(distinct)])
     xb, y = gpu.Buffer.of(packs.reshape(-1)), gpu.Buffer(ncols * rows * 4)
