@@ -385,7 +385,8 @@ static bool gemm_tiled(const cj_gemv_args &a, int64_t &wgs) {
     const int64_t cus = std::max(1, g.cus), gx = ((int64_t)a.batch + 127) / 128, gy = (a.rows + 63) / 64;
     const int64_t rounds = (gx * gy + cus - 1) / cus;
     wgs = gx * (gy >= 8 ? (gy + 7) / 8 * 8 : gy);
-    if (wgs > 0x7fffffff || (a.type != CJ_Q6_K && gy > 65535)) return false;
+    // shapes past the other kernels' grids stay theirs to refuse
+    if (wgs > 0x7fffffff || (a.type == CJ_Q6_K ? (a.batch + 15) / 16 : gy) > 65535) return false;
     if (a.type == CJ_Q8_0) {
         const int64_t t64 = gy * (((int64_t)a.batch + 63) / 64);   // the other kernel's tiles
         if (t64 < 256 && a.batch <= 64) return a.rows * (((int64_t)a.batch + 31) / 32 * 32) > 2200 * cus * rounds;
