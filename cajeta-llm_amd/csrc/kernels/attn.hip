@@ -1650,28 +1650,84 @@ extern "C" __global__ void __launch_bounds__(64) cj_qkprep(cj_qkprep_args a) {
 // (q·scale rounded, then the dot), the running max from -1e30, a rescale
 // only where the maximum rises, out = acc·(1/l).
 //
-// Sixteen lanes own one (row, head): lane j holds q[16v+j]·scale and the
-// accumulators of dims 16v+j (v < 8) and forms the partial
-// Σ_v q[16v+j]·k[16v+j] in v order; the 16 partials fold by the fixed
-// pairwise tree in four DPP steps within the 16-lane row (quad xor 1, quad
-// xor 2, half-row mirror, row mirror: pairs, quads, halves, the whole — fp
-// addition commutes, so all 16 lanes end with the tree's bits). A workgroup
-// of 4 waves takes RB rows of one kv head, 16·NS (row, head) pairs (NS a
-// wave; a wave's four pairs share a row for G ≥ 4); each tile of TK
-// positions is staged once for all of them, as f32 in lane order
-// ([t][j][v], so a lane's 8 values are two 16-byte reads that all of a
-// wave's pairs share). The heaviest row blocks are dispatched first.
-template <int CTRL>
-DEV float dpp_rowf(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false)); }
+// Sixteen lanes own one (row, head): lane l holds q[16v+j]·scale and the
+// accumulators of dims 16v+j (v < 8), j = pf_part(l), and forms the partial
+// Σ_v q[16v+j]·k[16v+j] in v order. The reference's exps and maxima are one
+// a position, so positions go in runs of 16, one a lane:
+//   scores   the 16 lanes' partials of the run's 16 positions fold by the
+//            fixed pairwise tree (fp addition commutes), each level halving
+//            the positions a lane still holds, so lane l ends with the score
+//            of position j (15 adds a run, not 64); the lanes' order makes
+//            every level's partner one DPP operand away (quad xor 1, quad
+//            xor 2, half-row mirror, row rotation by 8);
+//   max      a prefix maximum over the 16 lanes, from the running maximum;
+//   exps     lane i: position i's weight and, where it raises the maximum,
+//            its rescale: one exp for the four pairs' 16 positions;
+//   update   in position order, each position's weight broadcast in its row.
+// A workgroup of 4 waves takes RB rows of one kv head, 16·NS (row, head)
+// pairs (NS a wave; a wave's four pairs share a row for G ≥ 4); each tile of
+// TK positions is staged once for all of them as halves in lane order
+// ([t][j][v]: a lane's 8 values are one 16-byte read that all of a wave's
+// pairs share), the next tile's loads in flight meanwhile. The heaviest row
+// blocks are dispatched first.
+//
+// Bound by VALU issue: the order fixes 8 multiplies and 7 adds a lane for the
+// partial, 8 and 8 for the update and one add for the sum.
+// Measured (MI355X): eight ragged 1100-token prompts and 32 steps on two
+// 8B-shape layers 38.1 → 34.4 ms a pass; a 512-row chunk's launch with 32/8
+// heads 86 us at position 0, 190–273 at 512 (an exp a position and pair on
+// all 16 lanes, f32 tiles: 161 at position 0).
+template <int CTRL, int BANKS = 0xF>
+DEV float dpp_rowf(float old, float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL, 0xF, BANKS, false));
+}
+// lane l of 16 ↔ partial j: l = (j & 3) ^ (j & 4 ? 7 : 0) ^ (j & 8) and back
+DEV int pf_part(int l) { return (l & 4) ? l ^ 3 : l; }
+
+// One level of the fold: n positions' partials a lane become n / 2. A lane
+// with `up` keeps the odd half, and sends its partner the other.
+template <int CTRL, int N>
+DEV void pf_fold(float (&d)[16], bool up) {
+#pragma unroll
+    for (int i = 0; i < N / 2; i++) {
+        const float lo = d[2 * i], hi = d[2 * i + 1];
+        const float keep = up ? hi : lo, give = up ? lo : hi;
+        d[i] = __fadd_rn(keep, dpp_rowf<CTRL>(0.0f, give));
+    }
+}
+
+// Positions I.. of a run into the accumulators, in order. MASK: only where
+// the pair's lanes see the position.
+template <int I, bool MASK>
+DEV void pf_update(const uint8_t *vp, float pw, float cf, uint32_t ups, uint32_t lives, float (&acc)[8], float &l) {
+    if constexpr (I < 16) {
+        const uint4 vv = *(const uint4 *)(vp + 256 * I);
+        const float w = dpp_rowf<0x150 + I>(0.0f, pw);
+        if (!MASK || ((lives >> I) & 1)) {
+            if ((ups >> I) & 1) {   // a pair of the wave rescales (by 1 where its maximum stands)
+                const float c = dpp_rowf<0x150 + I>(0.0f, cf);
+#pragma unroll
+                for (int v = 0; v < 8; v++) acc[v] = __fmul_rn(acc[v], c);
+                l = __fmul_rn(l, c);
+            }
+            l = __fadd_rn(l, w);
+            const uint32_t vw[4] = {vv.x, vv.y, vv.z, vv.w};
+#pragma unroll
+            for (int v = 0; v < 8; v++)
+                acc[v] = __fadd_rn(acc[v], (v & 1) ? mul_h16hi(vw[v >> 1], w) : mul_h16lo(vw[v >> 1], w));
+        }
+        pf_update<I + 1, MASK>(vp, pw, cf, ups, lives, acc, l);
+    }
+}
 
 template <int G>
 DEV void prefill_body(const cj_attn_args &a) {
     constexpr int HD = 128, TK = 32, NS = G >= 8 ? G / 4 : 1, RB = 16 * NS / G;
-    __shared__ __align__(16) float kl[TK][16][8];
-    __shared__ __align__(16) float vl[TK][16][8];
+    __shared__ __align__(16) uint8_t kl[2][TK][256];
+    __shared__ __align__(16) uint8_t vl[2][TK][256];
     __shared__ uint64_t etab[32];
     cj_exp_table(etab);   // visible after the first tile's barrier
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, j = lane & 15, grp = lane >> 4;
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, l16 = lane & 15, grp = lane >> 4, j = pf_part(l16);
     const int nblk = (a.nrows + RB - 1) / RB;
     const int kvh = (int)(blockIdx.x % a.n_kv), rb = nblk - 1 - (int)(blockIdx.x / a.n_kv);
     const int slot = a.rowtab[0];
@@ -1706,63 +1762,85 @@ DEV void prefill_body(const cj_attn_args &a) {
         m[s] = -1.0e30f;
         l[s] = 0.0f;
     }
-    for (int tb = lo; tb < hi; tb += TK) {
-        const int nt = hi - tb < TK ? hi - tb : TK;
-        __syncthreads();   // the previous tile's reads are done
-        // stage: chunk c = 8 halves (dims 8m .. 8m+7) of key c/16; dim d goes
-        // to lane d & 15, slot d >> 4
-        uint4 kr[2], vr[2];
+    // stage: thread (key t / 8, dims 16v + 2·(t % 8) and the next); a key past
+    // the range repeats its last
+    uint32_t kr[8], vr[8];
+    auto fetch = [&](int tb) {
+        const int pos = min(tb + (t >> 3), hi - 1);
+        const int page = a.pgtab[pg_base + (pos >> 6)];
+        const int64_t off = (((int64_t)page * a.n_kv + kvh) * 64 + (pos & 63)) * HD + 2 * (t & 7);
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int c = t + 256 * i, kk = c >> 4, mp = c & 15;
-            const int pos = tb + (kk < nt ? kk : nt - 1);
-            const int page = a.pgtab[pg_base + (pos >> 6)];
-            const int64_t off = (((int64_t)page * a.n_kv + kvh) * 64 + (pos & 63)) * HD + 8 * mp;
-            kr[i] = *(const uint4 *)(a.kc + off);
-            vr[i] = *(const uint4 *)(a.vc + off);
+        for (int v = 0; v < 8; v++) {
+            kr[v] = *(const uint32_t *)(a.kc + off + 16 * v);
+            vr[v] = *(const uint32_t *)(a.vc + off + 16 * v);
         }
+    };
+    auto store = [&](int buf) {
+        auto put = [&](uint8_t *dst, const uint32_t (&w)[8]) {
+            u32x4 e, o;
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int c = t + 256 * i, kk = c >> 4, mp = c & 15;
-            const int j0 = (mp & 1) * 8, v0 = mp >> 1;
-            const uint32_t kw[4] = {kr[i].x, kr[i].y, kr[i].z, kr[i].w}, vw[4] = {vr[i].x, vr[i].y, vr[i].z, vr[i].w};
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                kl[kk][j0 + e][v0] = h2f(kw[e >> 1] >> (16 * (e & 1)));
-                vl[kk][j0 + e][v0] = h2f(vw[e >> 1] >> (16 * (e & 1)));
+            for (int i = 0; i < 4; i++) {
+                e[i] = __builtin_amdgcn_perm(w[2 * i + 1], w[2 * i], 0x05040100u);
+                o[i] = __builtin_amdgcn_perm(w[2 * i + 1], w[2 * i], 0x07060302u);
             }
-        }
-        __syncthreads();
-        for (int tt = 0; tt < nt; tt++) {
-            const int tp = tb + tt;
-            const float4 ka = *(const float4 *)&kl[tt][j][0], kb = *(const float4 *)&kl[tt][j][4];
-            const float4 va = *(const float4 *)&vl[tt][j][0], vb = *(const float4 *)&vl[tt][j][4];
-            const float kf[8] = {ka.x, ka.y, ka.z, ka.w, kb.x, kb.y, kb.z, kb.w};
-            const float vf[8] = {va.x, va.y, va.z, va.w, vb.x, vb.y, vb.z, vb.w};
+            *(u32x4 *)dst = e;
+            *(u32x4 *)(dst + 16) = o;
+        };
+        put(&kl[buf][t >> 3][32 * (t & 7)], kr);
+        put(&vl[buf][t >> 3][32 * (t & 7)], vr);
+    };
+    if (lo < hi) {
+        fetch(lo);
+        store(0);
+    }
+    __syncthreads();
+    int buf = 0;
+    for (int tb = lo; tb < hi; tb += TK, buf ^= 1) {
+        if (tb + TK < hi) fetch(tb + TK);
+#pragma unroll 1
+        for (int h = 0; h < TK; h += 16) {
+            const int p0 = tb + h;
 #pragma unroll
             for (int s = 0; s < NS; s++) {
-                if (tp >= c0[s] && tp < c1[s]) {
-                    float d = __fmul_rn(qv[s][0], kf[0]);
+                const bool live = p0 + l16 >= c0[s] && p0 + l16 < c1[s];
+                const uint64_t lives = __ballot(live);
+                if (!lives) continue;
+                float d[16];
 #pragma unroll
-                    for (int v = 1; v < 8; v++) d = __fadd_rn(d, __fmul_rn(qv[s][v], kf[v]));
-                    d = __fadd_rn(d, dpp_rowf<0xB1>(d));    // quad xor 1: the pairs
-                    d = __fadd_rn(d, dpp_rowf<0x4E>(d));    // quad xor 2: the quads
-                    d = __fadd_rn(d, dpp_rowf<0x141>(d));   // half-row mirror: the halves of 8
-                    d = __fadd_rn(d, dpp_rowf<0x140>(d));   // row mirror: the 16
-                    if (d > m[s]) {
-                        const float c = cj_expf(m[s] - d, etab);
+                for (int p = 0; p < 16; p++) {
+                    const uint4 kk = *(const uint4 *)&kl[buf][h + p][16 * j];
+                    const uint32_t kw[4] = {kk.x, kk.y, kk.z, kk.w};
+                    d[p] = mul_h16lo(kw[0], qv[s][0]);
 #pragma unroll
-                        for (int v = 0; v < 8; v++) acc[s][v] = __fmul_rn(acc[s][v], c);
-                        l[s] = __fmul_rn(l[s], c);
-                        m[s] = d;
-                    }
-                    const float pw = cj_expf(d - m[s], etab);
-                    l[s] = __fadd_rn(l[s], pw);
-#pragma unroll
-                    for (int v = 0; v < 8; v++) acc[s][v] = __fadd_rn(acc[s][v], __fmul_rn(vf[v], pw));
+                    for (int v = 1; v < 8; v++)
+                        d[p] = __fadd_rn(d[p], (v & 1) ? mul_h16hi(kw[v >> 1], qv[s][v]) : mul_h16lo(kw[v >> 1], qv[s][v]));
                 }
+                pf_fold<0xB1, 16>(d, j & 1);    // quad xor 1: the pairs
+                pf_fold<0x4E, 8>(d, j & 2);     // quad xor 2: the quads
+                pf_fold<0x141, 4>(d, j & 4);    // half-row mirror: the halves of 8
+                pf_fold<0x128, 2>(d, j & 8);    // row rotation by 8: the 16
+                // lane l holds position pf_part(l): banks 1 and 3 reversed give position l
+                const float sc = dpp_rowf<0x1B, 0xA>(d[0], d[0]);
+                float pm = live ? sc : -3.0e38f;
+                pm = fmaxf(pm, dpp_rowf<0x111>(pm, pm));
+                pm = fmaxf(pm, dpp_rowf<0x112>(pm, pm));
+                pm = fmaxf(pm, dpp_rowf<0x114>(pm, pm));
+                pm = fmaxf(pm, dpp_rowf<0x118>(pm, pm));
+                const float inc = fmaxf(m[s], pm), exc = dpp_rowf<0x111>(m[s], inc);
+                const bool up = live && sc > exc;
+                const uint64_t ub = __ballot(up);
+                float cf = 1.0f;
+                if (ub) cf = up ? cj_expf(exc - sc, etab) : 1.0f;
+                const float pw = cj_expf(sc - inc, etab);
+                m[s] = dpp_rowf<0x15F>(0.0f, inc);
+                const uint32_t u2 = (uint32_t)ub | (uint32_t)(ub >> 32), ups = (u2 | (u2 >> 16)) & 0xFFFFu;
+                const uint8_t *vp = &vl[buf][h][16 * j];
+                if (lives == ~0ull) pf_update<0, false>(vp, pw, cf, ups, 0u, acc[s], l[s]);
+                else pf_update<0, true>(vp, pw, cf, ups, (uint32_t)(lives >> (16 * grp)) & 0xFFFFu, acc[s], l[s]);
             }
         }
+        if (tb + TK < hi) store(buf ^ 1);
+        __syncthreads();
     }
 #pragma unroll
     for (int s = 0; s < NS; s++) {

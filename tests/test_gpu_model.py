@@ -373,6 +373,25 @@ def test_prefill_attend_query_groups(gpu, heads, kv):
     assert run_pair.bit_identical, err
 
 
+@pytest.mark.parametrize("heads,kv,swa,chunk,n", [(8, 2, 40, 37, 150), (16, 2, 100, 19, 150), (4, 4, 7, 50, 120),
+                                                  (8, 4, 16, 2, 40), (8, 2, 0, 512, 15), (8, 2, 0, 512, 34)])
+def test_prefill_attend_runs(gpu, heads, kv, swa, chunk, n):
+    """The prefill attend's runs of 16 positions off their edges: windows that
+    start and chunks that end inside a run, rows of a wave that see different
+    positions, a prompt shorter than a run; bit for bit."""
+    say("prefill attend runs", heads, kv, swa, chunk, n)
+    name = "t_pfr%d_%d_%d" % (heads, kv, chunk)
+    spec = "layers=2;hidden=1024;heads=%d;kv=%d;hd=128;ffn=1024;vocab=2048;eps=1e-5;theta=10000;" \
+           "wtype=q8_0;head=q8_0;embd=q8_0;ctx=256%s" % (heads, kv, ";swa=%d" % swa if swa else "")
+    path, img = synth(gpu, spec, name, 31 + n)
+    rng = np.random.default_rng(heads + chunk)
+    prompt = rng.integers(0, 2048, n).tolist()
+    g, o, err = run_pair(gpu, path, img, prompt, 2, 256, chunk=chunk)
+    gpu.image_free(name)
+    assert g == o
+    assert run_pair.bit_identical, err
+
+
 def test_c4_shape_q8_0_two_layers_greedy_parity(gpu):
     """Benchmark configuration C4's Q8_0 weights on the 8B shapes, at two layers."""
     say("model c4x2")
