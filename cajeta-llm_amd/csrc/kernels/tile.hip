@@ -654,3 +654,177 @@ extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_pe
     }
     mt_write(a, r0 + W.row, c0 + 32 * (W.wave & 3) + 4 * W.hf, W.acc);
 }
+
+// ------------------------------------------------- MXFP4 experts of many rows
+
+// A workgroup (row tile, expert) over the selections of the expert, as
+// moe_grp_body, its products on the int8 matrix cores. A row value is the sum
+// of 32 partials by the half-wave's butterfly (16, 8, 4, 2, 1), partial L
+// holding the blocks L, L + 32, L + 64 in order. Blocks ≡ j mod 8 are wave
+// j's: the partials j, j + 8, j + 16, j + 24, which the butterfly's first two
+// levels join; the waves' values meet in LDS for the other three. The eight
+// waves read the same 128-byte lines of the weight rows (16 bytes a block) and
+// of the packs together. A wave keeps its weights decoded in registers over
+// the members, which go 32 a chunk; the next chunk's codes are requested
+// before the current one's epilogue.
+//
+// Bound by VALU issue: four steps an output and block (the sum's conversion,
+// the two scales, the add), where the dot4 kernel spends twelve.
+// Measured (MI355X, 32 experts of 2880 × 2880, 4 a row): 512 rows gate|up
+// 1056 → 459 us, down 598 → 276; 128 rows 322 → 270, 186 → 155. At few rows
+// the weights' decode and scale table (about 150 us for all the experts)
+// bound it.
+template <int EPI, int KB>
+DEV void moe_tile_body(const cj_moe_grp_args &a) {
+    constexpr int RT = EPI == CJ_EPI_GLU ? 2 : 1, ROWS = 32 * RT, NM = 4 * KB, WS = ROWS + 4;
+    __shared__ __align__(16) float ws[32 * KB * WS];
+    __shared__ __align__(16) float part[8 * RT * 1024];   // [wave][tile][16 rows' quads][64 lanes][4]
+    __shared__ float act[32 * 33];
+    __shared__ int mi[3][32];   // a wave may still read the chunk before while another requests the next
+    const int e = blockIdx.y;
+    const int c = a.cnt[e];
+    if (c == 0) return;
+    const int t = threadIdx.x, lane = t & 63, m32 = lane & 31, hf = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nb = (int)(a.cols / 32);
+    const uint8_t *W = a.w + (int64_t)e * a.expert_bytes;
+    const int64_t row0 = (int64_t)blockIdx.x * ROWS;
+    const int32_t *mem = a.mem + (int64_t)e * a.cap;
+
+    i32x4 x[NM];
+    float xs[NM];
+    auto fetch = [&](int j0, int buf) {
+        const int me = mem[min(j0 + m32, c - 1)];
+        if (t < 32) mi[buf][t] = me;
+        const uint8_t *row = a.xp + (int64_t)(me / a.x_per) * a.xp_stride + 32 * wave;
+#pragma unroll
+        for (int k = 0; k < NM; k++) {
+            const int q = min(8 * k + wave, nb - 1) >> 3;
+            x[k] = *(const i32x4 *)(row + q * 320 + 16 * hf);
+            xs[k] = *(const float *)(row + q * 320 + 288 - 28 * wave);
+        }
+    };
+    fetch(0, 0);
+    i32x4 w[RT][NM];
+#pragma unroll
+    for (int r = 0; r < RT; r++) {
+        const uint8_t *wr = W + min(row0 + 32 * r + m32, a.rows - 1) * a.row_bytes;
+#pragma unroll
+        for (int k = 0; k < NM; k++) w[r][k] = *(const i32x4 *)(wr + 16 * min(8 * k + wave, nb - 1));
+    }
+    for (int i = t; i < ROWS * 32 * KB; i += 512) {
+        const int r = i / (32 * KB), b = i % (32 * KB);
+        ws[b * WS + r] = b < nb ? mxfp4_scale(W[min(row0 + r, a.rows - 1) * a.row_bytes + 16 * nb + b]) : 0.0f;
+    }
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+        for (int k = 0; k < NM; k++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) w[r][k][i] = (int)e2m1_x4((uint32_t)w[r][k][i] >> (4 * hf));
+    __syncthreads();
+
+    int buf = 0;
+    for (int j0 = 0; j0 < c; j0 += 32, buf = buf == 2 ? 0 : buf + 1) {
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            // the chains of partials 0, 2, 1, 3 (in units of 8), their blocks in order
+            f32x16 s, u, v;
+            i32x16 Z;   // (the conversions cost less than 16 registers for mt_magic, which would spill)
+#pragma unroll
+            for (int i = 0; i < 16; i++) { s[i] = u[i] = v[i] = 0.0f; Z[i] = 0; }
+#pragma unroll
+            for (int f = 0; f < NM; f++) {
+                constexpr int ORDER[4] = {0, 2, 1, 3};
+                const int n = 4 * (f % KB) + ORDER[f / KB], b = 8 * n + wave;
+                f32x16 &p = f / KB == 0 ? s : f / KB == 3 ? v : u;
+                if (f == 2 * KB) {
+#pragma unroll
+                    for (int i = 0; i < 16; i++) { s[i] = __fadd_rn(s[i], u[i]); u[i] = 0.0f; }
+                }
+                if (b < nb) {
+                    const i32x16 d = mt_dot(w[r][n], x[n], Z);
+                    const float *wp = ws + b * WS + 32 * r + 4 * hf;
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const f32x4 wv = *(const f32x4 *)(wp + 8 * q);
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+                            const float term = __fmul_rn(__fmul_rn((float)d[4 * q + k], wv[k]), xs[n]);
+                            p[4 * q + k] = __fadd_rn(p[4 * q + k], term);
+                        }
+                    }
+                }
+                // the next product waits for this fold (as in the Q4_K kernel)
+                if (f + 1 < NM) asm volatile("" : "+v"(x[4 * ((f + 1) % KB) + ORDER[(f + 1) / KB]]), "+v"(p));
+            }
+            float *pp = part + (wave * RT + r) * 1024 + 4 * lane;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                f32x4 o;
+#pragma unroll
+                for (int k = 0; k < 4; k++) o[k] = __fadd_rn(s[4 * q + k], __fadd_rn(u[4 * q + k], v[4 * q + k]));
+                *(f32x4 *)(pp + 256 * q) = o;
+            }
+        }
+        if (j0 + 32 < c) fetch(j0 + 32, buf == 2 ? 0 : buf + 1);
+        lds_barrier();
+        const int nc = min(32, c - j0);
+        if (t < 256 * RT) {
+            // thread (tile t / 256, quad, lane): four rows of one member
+            f32x4 p[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) p[k] = *(const f32x4 *)(part + (k * RT + (t >> 8)) * 1024 + 4 * (t & 255));
+            f32x4 o;
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                o[k] = __fadd_rn(__fadd_rn(__fadd_rn(p[0][k], p[4][k]), __fadd_rn(p[2][k], p[6][k])),
+                                 __fadd_rn(__fadd_rn(p[1][k], p[5][k]), __fadd_rn(p[3][k], p[7][k])));
+            const int rl = 32 * (t >> 8) + 8 * ((t >> 6) & 3) + 4 * hf;
+            if (EPI == CJ_EPI_GLU) {
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    const int64_t ai = (row0 + rl) / 2 + k;
+                    act[m32 * 33 + rl / 2 + k] =
+                        m32 < nc && ai < a.act_n ? glu_value(a.glu_form, ai, a.act_n, o[2 * k], o[2 * k + 1]) : 0.0f;
+                }
+            } else if (m32 < nc && row0 + rl < a.rows) {   // (rows are a multiple of four)
+                *(f32x4 *)(a.y + (int64_t)mi[buf][m32] * a.y_stride + row0 + rl) = o;
+            }
+        }
+        lds_barrier();
+        if (EPI == CJ_EPI_GLU) {
+            // the 32 values of a member are one 32-block of its activation
+            const int64_t ab = row0 / ROWS;
+            const int o = t & 31;
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const int jj = 16 * k + (t >> 5);
+                const float v = act[jj * 33 + o];
+                const float bm = xmax32(fabsf(v));
+                const float inv = bm > 0.0f ? __fdiv_rn(127.0f, bm) : 0.0f;
+                const int q = round_away(__fmul_rn(v, inv));
+                const int sq = xsum32_i(q);
+                if (jj < nc) {
+                    uint8_t *ob = a.outp + (int64_t)mi[buf][jj] * a.outp_stride + (ab >> 3) * 320;
+                    ob[(ab & 7) * 32 + o] = (uint8_t)(int8_t)q;
+                    if (o == 0) {
+                        *(int32_t *)(ob + 256 + 4 * (ab & 7)) = sq;
+                        *(float *)(ob + 288 + 4 * (ab & 7)) = __fdiv_rn(bm, 127.0f);
+                    }
+                }
+            }
+        }
+    }
+}
+#define MOE_TILE_KERNEL(E, EPI, KB)                                                                                          \
+    extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))                                \
+        cj_moe_t_##E##_k##KB(cj_moe_grp_args a) {                                                                            \
+        moe_tile_body<EPI, KB>(a);                                                                                           \
+    }
+MOE_TILE_KERNEL(g, CJ_EPI_GLU, 1)
+MOE_TILE_KERNEL(g, CJ_EPI_GLU, 2)
+MOE_TILE_KERNEL(g, CJ_EPI_GLU, 3)
+MOE_TILE_KERNEL(s, CJ_EPI_STORE, 1)
+MOE_TILE_KERNEL(s, CJ_EPI_STORE, 2)
+MOE_TILE_KERNEL(s, CJ_EPI_STORE, 3)

@@ -973,6 +973,17 @@ int Engine::rows_moe(const Layer &L, int n) {
         const char *rcv = getenv("CJ_GRP_RC");   // "<rw><cc>": 14, 24
         auto grp = [&](const char *form, int grt, cj_moe_grp_args &q) {
             const int nbq = (int)(q.cols / 32), kb = std::min(4, std::max(1, (nbq + 31) / 32));
+            // the matrix-core tiles from 14 selections an expert on, and where
+            // a wave's decoded rows fit its registers (96 blocks). Measured
+            // (32 experts of 2880, 4 a row; dot4 kernel → tiles, gate|up + down,
+            // us): 64 rows 282 → 367, 96 rows 397 → 384, 128 rows 508 → 425,
+            // 300 rows 1062 → 550, 512 rows 1653 → 735
+            if (kb <= 3 && sels >= 14 * n_experts) {
+                char tname[32];
+                snprintf(tname, sizeof tname, "cj_moe_t_%s_k%d", form, kb);
+                const int64_t rows = *form == 'g' ? 64 : 32;
+                return launch2(tname, (uint32_t)((q.rows + rows - 1) / rows), (uint32_t)n_experts, 512, 0, q);
+            }
             const int cc = rcv && kb == 3 ? 4 : 16;
             const uint32_t lds = (uint32_t)(cc * ((q.cols + 15) & ~15) + cc * ((nbq + 3) & ~3) * 4 + grt * (cc + 1) * 4);
             char kname[48];

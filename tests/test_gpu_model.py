@@ -421,6 +421,26 @@ def test_c4_shape_q8_0_batched_decode_parity(gpu):
     assert err <= LOGIT_TOL and same
 
 
+@pytest.mark.parametrize("hidden,ffn,experts,used,n", [(512, 1056, 4, 2, 150), (2080, 512, 2, 1, 66), (1024, 2112, 3, 3, 33),
+                                                       (512, 32, 5, 2, 90)])
+def test_moe_expert_tiles(gpu, hidden, ffn, experts, used, n):
+    """MXFP4 experts of a prefill chunk on the matrix-core tiles: rows of one
+    to three sweeps of 32 blocks, ones that end inside a sweep and inside a
+    pack block among them, and members on either side of a chunk of 32; bit
+    for bit."""
+    say("moe expert tiles", hidden, ffn, experts, used, n)
+    name = "t_moet%d_%d" % (hidden, ffn)
+    spec = "layers=2;hidden=%d;heads=8;kv=2;hd=64;ffn=%d;vocab=2048;eps=1e-5;theta=150000;wtype=q8_0;head=q8_0;embd=q8_0;" \
+           "experts=%d;used=%d;expert_ffn=%d;expert_type=mxfp4;ctx=256" % (hidden, ffn, experts, used, ffn)
+    path, img = synth(gpu, spec, name, 7 + n)
+    rng = np.random.default_rng(hidden + n)
+    prompt = rng.integers(0, 2048, n).tolist()
+    g, o, err = run_pair(gpu, path, img, prompt, 2, 256)
+    gpu.image_free(name)
+    assert g == o
+    assert run_pair.bit_identical, err
+
+
 def test_c5_moe_shape_two_layers_greedy_parity(gpu):
     """Benchmark configuration C5's gpt-oss-20b shapes (d 2880, 64/8 heads of 64, 32
     MXFP4 experts top-4 of FFN 2880, alternating 128-window attention) at two
