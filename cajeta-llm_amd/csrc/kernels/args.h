@@ -252,6 +252,9 @@ typedef struct {
     int32_t *status;         // set to 1 when a row's logits are not finite (may be null)
 } cj_route_args;
 
+// The f32 router of many rows (rows of x and w are cols floats apart)
+typedef struct { const float *w, *x; float *y; int64_t cols; int32_t nrows, experts; } cj_rows_router_args;
+
 // The rows' expert selections grouped by expert (MoeFfn.forwardRowsZeroSync
 // reads each selected expert once for all the rows that chose it).
 typedef struct {

@@ -157,3 +157,61 @@ extern "C" __global__ void __launch_bounds__(256) cj_rows_pick(cj_rows_args a) {
         st->pos = pos + 1;
     }
 }
+
+// The router logits of many rows: y[r][e] = Σ_k w[e][k]·x[r][k], each product
+// and add rounded, k ascending from +0 — a lane an output, 16 rows × 16
+// experts a workgroup, both operands staged 64 columns a step (rows 68 floats
+// apart: 16 lanes' 16-byte reads of 16 rows fall on all banks once), the next
+// step's loads in flight. Bound by the chain's latency, which the outputs
+// share where a workgroup an output walked each alone.
+// Measured (MI355X, 32 experts × 2880): 33 us from 33 to 512 rows; a workgroup
+// an output took 25 us at 32 rows and 198 at 300.
+extern "C" __global__ void __launch_bounds__(256) cj_rows_router(cj_rows_router_args a) {
+    constexpr int KC = 64, S = KC + 4;
+    __shared__ __align__(16) float xt[2][16][S], wt[2][16][S];
+    const int t = threadIdx.x, lr = t >> 4, lc = 4 * (t & 15);
+    const int64_t r0 = (int64_t)blockIdx.x * 16;
+    const int e0 = (int)blockIdx.y * 16;
+    const float *xr = a.x + min(r0 + lr, (int64_t)a.nrows - 1) * a.cols;
+    const float *wr = a.w + (int64_t)min(e0 + lr, a.experts - 1) * a.cols;
+    float4 xv, wv;
+    auto fetch = [&](int64_t k) {
+        const int64_t c = min(k + lc, a.cols - 4);   // (past the row: staged, never read)
+        xv = *(const float4 *)(xr + c);
+        wv = *(const float4 *)(wr + c);
+    };
+    auto store = [&](int buf) {
+        *(float4 *)&xt[buf][lr][lc] = xv;
+        *(float4 *)&wt[buf][lr][lc] = wv;
+    };
+    fetch(0);
+    store(0);
+    __syncthreads();
+    float acc = 0.0f;
+    int buf = 0;
+    for (int64_t k = 0; k < a.cols; k += KC, buf ^= 1) {
+        if (k + KC < a.cols) fetch(k + KC);
+        const float *xp = xt[buf][t >> 4], *wp = wt[buf][t & 15];
+        const int n = (int)min((int64_t)KC, a.cols - k);
+        for (int c = 0; c < n; c += 32) {   // (columns are whole 32-element blocks)
+            float4 u[8], v[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                u[i] = *(const float4 *)(xp + c + 4 * i);
+                v[i] = *(const float4 *)(wp + c + 4 * i);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                acc = __fadd_rn(acc, __fmul_rn(v[i].x, u[i].x));
+                acc = __fadd_rn(acc, __fmul_rn(v[i].y, u[i].y));
+                acc = __fadd_rn(acc, __fmul_rn(v[i].z, u[i].z));
+                acc = __fadd_rn(acc, __fmul_rn(v[i].w, u[i].w));
+            }
+        }
+        if (k + KC < a.cols) store(buf ^ 1);
+        __syncthreads();
+    }
+    const int64_t r = r0 + (t >> 4);
+    const int e = e0 + (t & 15);
+    if (r < a.nrows && e < a.experts) a.y[r * a.experts + e] = acc;
+}

@@ -953,7 +953,13 @@ int Engine::rows_moe(const Layer &L, int n) {
         p.eps = eps; p.form = 0; p.per32 = L.gu_exps.type == CJ_Q8_0 || grouped; p.do_norm = 1;
         if ((rc = launch_norm_pack_rows(p, n))) return rc;
     }
-    {   // router logits of every row: the indirection's copies all read the router (expert_bytes 0)
+    if (n > 32 && hidden % 32 == 0 && L.router.row_bytes == (int64_t)hidden * 4) {
+        // one chain's latency whatever the rows; the other kernel's time grows
+        // with them (2880 × 32 experts: 14 us at 16 rows, 25 at 32, 198 at
+        // 300; this one 33)
+        cj_rows_router_args a{(const float *)L.router.p, r_xn, r_moe_logits, hidden, n, n_experts};
+        if ((rc = launch2("cj_rows_router", (uint32_t)((n + 15) / 16), (uint32_t)((n_experts + 15) / 16), 256, 0, a))) return rc;
+    } else {   // router logits of every row: the indirection's copies all read the router (expert_bytes 0)
         cj_gemv_args a{};
         a.w = (const uint8_t *)L.router.p; a.x = r_xn; a.y = r_moe_logits; a.rows = n_experts; a.cols = hidden;
         a.row_bytes = L.router.row_bytes; a.type = CJ_F32; a.pro = CJ_PRO_F32; a.epi = CJ_EPI_STORE; a.eps = eps;

@@ -500,7 +500,7 @@ int32_t cj_init(int32_t device) {
         "cj_gemm_q80_n2", "cj_gemm_q4k_n2", "cj_gemm_q80_n4", "cj_gemm_q6k_c4", "cj_gemm_q6k_c8", "cj_gemm_q6k_m16",
         "cj_gemm_sk_q80_n1", "cj_gemm_sk_q80_n2", "cj_gemm_sk_q4k_n1", "cj_gemm_t_q4k", "cj_gemm_t_q6k", "cj_gemm_t_q80",
         "cj_moe_t_g_k1", "cj_moe_t_g_k2", "cj_moe_t_g_k3", "cj_moe_t_s_k1", "cj_moe_t_s_k2", "cj_moe_t_s_k3",
-        "cj_rows_embed", "cj_rows_qkv", "cj_rows_glu", "cj_rows_argmax", "cj_rows_pick",
+        "cj_rows_embed", "cj_rows_router", "cj_rows_qkv", "cj_rows_glu", "cj_rows_argmax", "cj_rows_pick",
         "cj_attn_split_rows_h128_g4", "cj_attn_split_rows_h128_g8", "cj_attn_merge_rows",
         "cj_attn_prefill_h128_g1", "cj_attn_prefill_h128_g2", "cj_attn_prefill_h128_g4", "cj_attn_prefill_h128_g8",
         "cj_attn_scores_rows_h64", "cj_attn_scores_rows_h128", "cj_attn_combine_rows_h64", "cj_attn_combine_rows_h128",

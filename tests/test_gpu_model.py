@@ -426,8 +426,9 @@ def test_c4_shape_q8_0_batched_decode_parity(gpu):
 def test_moe_expert_tiles(gpu, hidden, ffn, experts, used, n):
     """MXFP4 experts of a prefill chunk on the matrix-core tiles: rows of one
     to three sweeps of 32 blocks, ones that end inside a sweep and inside a
-    pack block among them, and members on either side of a chunk of 32; bit
-    for bit."""
+    pack block among them, and members on either side of a chunk of 32; the
+    many-row router's tiles off their edges (33 rows, 2 to 5 experts, a last
+    step of 32 columns); bit for bit."""
     say("moe expert tiles", hidden, ffn, experts, used, n)
     name = "t_moet%d_%d" % (hidden, ffn)
     spec = "layers=2;hidden=%d;heads=8;kv=2;hd=64;ffn=%d;vocab=2048;eps=1e-5;theta=150000;wtype=q8_0;head=q8_0;embd=q8_0;" \
