@@ -929,6 +929,26 @@ int Engine::rows_pack(const float *x, int64_t n, int per32, int rows) {
     return launch("cj_pack_blocks", (uint32_t)((p.npad / 256 * rows + 3) / 4), 256, 0, p);
 }
 
+// Whether cj_rows_router takes n rows' router product. It is one chain of
+// `cols` adds whatever the rows and experts (2 + cols / 93 us); the f32 GEMV
+// takes a round of workgroups at a time, a workgroup an output up to 64
+// experts (two a CU, one where the staged row passes 4096 columns; 4.3 + cols
+// / 390 us a round) and one 32 experts above (one a CU; 12.5 + cols / 300).
+// Measured on 256 CUs (us, GEMV → tiles): 2880 columns: 8 experts × 64 rows
+// 13 → 33 stays, × 256 47 → 33; 32 × 33 32 → 33 stays, × 64 47 → 33; 128 × 64
+// 22 → 33 stays, × 96 41 → 33; 512 columns: 4 × 64 6 → 7 stays, 32 × 64 23 →
+// 7; 7168 columns: 8 × 96 63 → 79 stays, 32 × 64 162 → 79. Over 2–256 experts
+// × 33–512 rows × 512–7168 columns the kernel taken is within 7% (0.5 us) of
+// the faster one. A decode step's up to 32 rows keep the GEMV.
+static bool rows_router_tiled(int64_t cols, int64_t experts, int64_t n) {
+    if (n <= 32) return false;
+    const bool one = experts <= 64;
+    const int64_t wgs = one ? n * experts : n * ((experts + 31) / 32);
+    const int64_t slots = (int64_t)std::max(1, device_cus()) * (one && cols <= 4096 ? 2 : 1);
+    const int64_t round_us = one ? 4300 + 1000 * cols / 390 : 12500 + 1000 * cols / 300;   // (thousandths)
+    return (wgs + slots - 1) / slots * round_us > 2000 + 1000 * cols / 93;
+}
+
 // The MoE FFN of n rows (MoeFfn.forwardRowsZeroSync, model/MoeFfn.cajeta:1559
 // and its comment at :1510-1515: one router product and one top-k over the
 // rows, one indirected product per expert bank over every row's
@@ -953,10 +973,7 @@ int Engine::rows_moe(const Layer &L, int n) {
         p.eps = eps; p.form = 0; p.per32 = L.gu_exps.type == CJ_Q8_0 || grouped; p.do_norm = 1;
         if ((rc = launch_norm_pack_rows(p, n))) return rc;
     }
-    if (n > 32 && hidden % 32 == 0 && L.router.row_bytes == (int64_t)hidden * 4) {
-        // one chain's latency whatever the rows; the other kernel's time grows
-        // with them (2880 × 32 experts: 14 us at 16 rows, 25 at 32, 198 at
-        // 300; this one 33)
+    if (hidden % 32 == 0 && L.router.row_bytes == (int64_t)hidden * 4 && rows_router_tiled(hidden, n_experts, n)) {
         cj_rows_router_args a{(const float *)L.router.p, r_xn, r_moe_logits, hidden, n, n_experts};
         if ((rc = launch2("cj_rows_router", (uint32_t)((n + 15) / 16), (uint32_t)((n_experts + 15) / 16), 256, 0, a))) return rc;
     } else {   // router logits of every row: the indirection's copies all read the router (expert_bytes 0)

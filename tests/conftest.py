@@ -27,3 +27,22 @@ def O():
 def gpu(pkg):
     pkg.native.init(0)
     return pkg
+
+
+@pytest.fixture
+def launched(gpu):
+    """launched(f): f()'s result and the names of the kernels that this thread launched meanwhile."""
+    import ctypes
+    lib = gpu.native.lib()
+    names = lib._ZN2cj12launch_namesEv
+    names.restype = ctypes.c_char_p
+
+    def record(f):
+        lib._ZN2cj18launch_names_resetEv()
+        try:
+            out = f()
+        finally:
+            seen = names().decode().split(" + ")
+        return out, seen
+
+    return record

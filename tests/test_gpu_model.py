@@ -426,9 +426,8 @@ def test_c4_shape_q8_0_batched_decode_parity(gpu):
 def test_moe_expert_tiles(gpu, hidden, ffn, experts, used, n):
     """MXFP4 experts of a prefill chunk on the matrix-core tiles: rows of one
     to three sweeps of 32 blocks, ones that end inside a sweep and inside a
-    pack block among them, and members on either side of a chunk of 32; the
-    many-row router's tiles off their edges (33 rows, 2 to 5 experts, a last
-    step of 32 columns); bit for bit."""
+    pack block among them, and members on either side of a chunk of 32; bit
+    for bit."""
     say("moe expert tiles", hidden, ffn, experts, used, n)
     name = "t_moet%d_%d" % (hidden, ffn)
     spec = "layers=2;hidden=%d;heads=8;kv=2;hd=64;ffn=%d;vocab=2048;eps=1e-5;theta=150000;wtype=q8_0;head=q8_0;embd=q8_0;" \
@@ -440,6 +439,28 @@ def test_moe_expert_tiles(gpu, hidden, ffn, experts, used, n):
     gpu.image_free(name)
     assert g == o
     assert run_pair.bit_identical, err
+
+
+@pytest.mark.parametrize("hidden,experts,used,n,etype,tiled", [(2080, 8, 2, 64, "mxfp4", False), (512, 4, 2, 64, "q8_0", False),
+                                                               (2080, 40, 2, 66, "mxfp4", True), (512, 130, 2, 33, "mxfp4", True),
+                                                               (1024, 17, 1, 81, "q8_0", True)])
+def test_moe_router_by_work(gpu, launched, hidden, experts, used, n, etype, tiled):
+    """The many-row router's tiles take a chunk where rows times experts fill
+    more rounds of the f32 GEMV than the tiles' one chain costs, and the GEMV
+    the others; the tiles off their edges (rows and experts that are not whole
+    16s, a last step of 32 columns); bit for bit either way."""
+    say("moe router", hidden, experts, used, n, etype)
+    name = "t_moer%d_%d" % (hidden, experts)
+    spec = "layers=2;hidden=%d;heads=8;kv=2;hd=64;ffn=32;vocab=1024;eps=1e-5;theta=150000;wtype=q8_0;head=q8_0;embd=q8_0;" \
+           "experts=%d;used=%d;expert_ffn=32;expert_type=%s;ctx=256" % (hidden, experts, used, etype)
+    path, img = synth(gpu, spec, name, 11 + n)
+    rng = np.random.default_rng(hidden + n)
+    prompt = rng.integers(0, 1024, n).tolist()
+    (g, o, err), kernels = launched(lambda: run_pair(gpu, path, img, prompt, 2, 256))
+    gpu.image_free(name)
+    assert g == o
+    assert run_pair.bit_identical, err
+    assert ("cj_rows_router" in kernels) == tiled, kernels
 
 
 def test_c5_moe_shape_two_layers_greedy_parity(gpu):
