@@ -362,21 +362,28 @@ GemvPlan plan_gemv(int type, int64_t rows, int64_t cols, int target, int pro, in
 
 bool gemm_supported(int type) { return type == CJ_Q8_0 || type == CJ_Q4_K || type == CJ_Q6_K; }
 
-// The 64-row × 128-column tile kernels (tile.hip) take about 2.05 us a
-// 256-element block and round of tiles over the CUs, however full the tiles
-// are. Their lines, measured on 256 CUs (us, 4096 columns of weights
-// unless named; other kernel → tile kernel):
+// The 64-row × 128-column tile kernels (tile.hip) take a round of tiles over
+// the CUs at a time, however full the tiles are (about 4 us and 1.9 us a
+// 256-element block; a 56-block row 98–114). Their lines, measured on 256 CUs
+// (us, 4096 columns of weights unless named; other kernel → tile kernel):
 //  - Q4_K: where the 64 × 32 tiles of the other kernel are more than one a CU
-//    for each round (4096 × 128: 31.5 → 34.2 stays; 6144 × 96: 43.9 → 33.3;
-//    4096 × 512: 75.9 → 34.2; 28672 × 17, two rounds: 45.8 → 65.9 stays,
-//    × 33: 84.2 → 66.8);
+//    for each round (4096 × 128: 31.5 → 34.2 stays; 4096 × 512: 75.9 → 34.2;
+//    28672 × 17, two rounds: 45.8 → 65.9 stays, × 33: 84.2 → 66.8), and by
+//    more the fewer blocks the rows have (the tiles' 4 us): of the other
+//    kernel's rounds w and these ones r, w + 0.5 ≥ r·(2.8 − blocks / 8)
+//    (20000 × 48, w 3 and r 2: of 512 columns 11.2 → 14.8 stays, 2048 36.9 →
+//    37.6 stays, 3072 54.8 → 51.8; 14336 × 33, 2 and 1: of 512 columns 7.5 →
+//    8.1 stays, 1024 12.5 → 12.2). Over 3038 shapes (64–32884 rows, 256–14336
+//    columns, 17–512 activations) the tiles are nowhere taken where they are
+//    more than 3.5% slower;
 //  - Q6_K: where rows × columns (in 16s) pass 1200 a CU for each round, the
 //    other kernel's 30 us (2048 × 128: 29.6 → 32.7 stays; 6144 × 64: 42.5 →
 //    32.4; 28672 × 17: 81 → 64; 4096 × 512: 209 → 35.5);
 //  - Q8_0, above 32 columns: against the split-K kernel where rows × columns
 //    (in 32s) pass 2200 a CU for each round (4096 × 64: 15.6 → 34 stays;
 //    14336 × 33: 48 → 34.5); against the 64 × 64 tiles in one round always
-//    (4096 × 512: 52 → 33; 14336 × 128: 51 → 36), in more where those tiles
+//    (4096 × 512: 52 → 33; 14336 × 128: 51 → 36; also where they are few:
+//    256 × 65, four tiles, 36.6 → 30.9), in more where those tiles
 //    pass 1.37 a CU for each round (14336 × 512, four rounds: 169 → 131.5).
 static bool gemm_tiled(const cj_gemv_args &a, int64_t &wgs) {
     if ((a.type != CJ_Q4_K && a.type != CJ_Q6_K && a.type != CJ_Q8_0) || a.batch <= (a.type == CJ_Q8_0 ? 32 : 16)) return false;
@@ -392,7 +399,10 @@ static bool gemm_tiled(const cj_gemv_args &a, int64_t &wgs) {
         if (t64 < 256 && a.batch <= 64) return a.rows * (((int64_t)a.batch + 31) / 32 * 32) > 2200 * cus * rounds;
         return rounds == 1 || 8 * t64 > 11 * cus * rounds;
     }
-    if (a.type == CJ_Q4_K) return gy * (((int64_t)a.batch + 31) / 32) > cus * rounds;
+    if (a.type == CJ_Q4_K) {
+        const int64_t t32 = gy * (((int64_t)a.batch + 31) / 32);
+        return t32 > cus * rounds && 16 * ((t32 + cus - 1) / cus) + 8 >= rounds * (45 - a.cols / 128);
+    }
     return a.rows * (((int64_t)a.batch + 15) / 16 * 16) > 1200 * cus * rounds;
 }
 
