@@ -381,7 +381,9 @@ bool gemm_supported(int type) { return type == CJ_Q8_0 || type == CJ_Q4_K || typ
 //    32.4; 28672 × 17: 81 → 64; 4096 × 512: 209 → 35.5);
 //  - Q8_0, above 32 columns: against the split-K kernel where rows × columns
 //    (in 32s) pass 2200 a CU for each round (4096 × 64: 15.6 → 34 stays;
-//    14336 × 33: 48 → 34.5); against the 64 × 64 tiles in one round always
+//    14336 × 33: 48 → 34.5), 2700 where rows are wider than 8192 columns
+//    (of 14336 columns 9216 × 33: 103 → 110 stays, 11264 × 33: 123 → 111);
+//    against the 64 × 64 tiles in one round always
 //    (4096 × 512: 52 → 33; 14336 × 128: 51 → 36; also where they are few:
 //    256 × 65, four tiles, 36.6 → 30.9), in more where those tiles
 //    pass 1.37 a CU for each round (14336 × 512, four rounds: 169 → 131.5).
@@ -396,7 +398,7 @@ static bool gemm_tiled(const cj_gemv_args &a, int64_t &wgs) {
     if (wgs > 0x7fffffff || (a.type == CJ_Q6_K ? (a.batch + 15) / 16 : gy) > 65535) return false;
     if (a.type == CJ_Q8_0) {
         const int64_t t64 = gy * (((int64_t)a.batch + 63) / 64);   // the other kernel's tiles
-        if (t64 < 256 && a.batch <= 64) return a.rows * (((int64_t)a.batch + 31) / 32 * 32) > 2200 * cus * rounds;
+        if (t64 < 256 && a.batch <= 64) return a.rows * (((int64_t)a.batch + 31) / 32 * 32) > (a.cols > 8192 ? 2700 : 2200) * cus * rounds;
         return rounds == 1 || 8 * t64 > 11 * cus * rounds;
     }
     if (a.type == CJ_Q4_K) {

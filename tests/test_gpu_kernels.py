@@ -727,29 +727,33 @@ def test_matmul_tile_kernels(gpu, O, name, ty, rows, cols, ncols):
         b.free()
 
 
-@pytest.mark.parametrize("rows,cols,ncols,tiled", [(20000, 512, 48, False), (14336, 512, 33, False), (14336, 1024, 33, True),
-                                                   (20000, 256, 96, False), (8200, 256, 127, True), (16330, 1024, 150, True)])
-def test_q4k_tile_line(gpu, O, launched, rows, cols, ncols, tiled):
-    """Q4_K products on both sides of the tile kernel's line, which rises as
-    rows get shorter (a tile's fixed time); bit for bit on either side."""
-    say("q4_k tile line", rows, cols, ncols)
+@pytest.mark.parametrize("ty,rows,cols,ncols,tiled", [(12, 20000, 512, 48, False), (12, 14336, 512, 33, False),
+                                                      (12, 14336, 1024, 33, True), (12, 20000, 256, 96, False),
+                                                      (12, 8200, 256, 127, True), (12, 16330, 1024, 150, True),
+                                                      (8, 9216, 14336, 33, False), (8, 11264, 14336, 33, True),
+                                                      (8, 9216, 4096, 33, True)])
+def test_tile_line(gpu, O, launched, ty, rows, cols, ncols, tiled):
+    """Products on both sides of the tile kernels' lines: Q4_K's rises as rows
+    get shorter (a tile's fixed time), Q8_0's against the split-K kernel with
+    wide rows; bit for bit on either side."""
+    say("tile line", ty, rows, cols, ncols)
     rng = np.random.default_rng(rows + cols + ncols)
-    raw = rand_blocks(O, O.Q4_K, rows * cols // 256, rng).reshape(-1)
+    raw = rand_blocks(O, ty, rows * cols // O.BLOCK[ty][0], rng).reshape(-1)
     lib = gpu.native.lib()
-    w = gpu.Buffer(lib.cj_prepared_row_bytes(O.Q4_K, cols) * rows)
+    w = gpu.Buffer(lib.cj_prepared_row_bytes(ty, cols) * rows)
     src = gpu.Buffer.of(raw)
-    gpu.native.check(lib.cj_prepare_weight(w.h, src.h, O.Q4_K, rows, cols), "prepare")
+    gpu.native.check(lib.cj_prepare_weight(w.h, src.h, ty, rows, cols), "prepare")
     distinct = 5                                    # later columns repeat them
-    packs = np.stack([O.q8k_pack(rng.standard_normal(cols).astype(np.float32)) for _ in range(distinct)])
-    refs = [O.matvec_packed(O.Q4_K, raw, rows, cols, p) for p in packs]
+    packs = np.stack([O.q8k_pack(rng.standard_normal(cols).astype(np.float32), per32=(ty == O.Q8_0)) for _ in range(distinct)])
+    refs = [O.matvec_packed(ty, raw, rows, cols, p) for p in packs]
     stride = packs.shape[1]
     xb, y = gpu.Buffer.of(packs[np.arange(ncols) % distinct].reshape(-1)), gpu.Buffer(ncols * rows * 4)
     _, kernels = launched(lambda: gpu.native.check(
-        lib.cj_matmul(O.Q4_K, y.h, w.h, xb.h, rows, cols, ncols, stride, rows, 0, 0), "matmul"))
+        lib.cj_matmul(ty, y.h, w.h, xb.h, rows, cols, ncols, stride, rows, 0, 0), "matmul"))
     got = y.download(np.float32, ncols * rows).reshape(ncols, rows)
     for c in range(ncols):
         assert np.array_equal(got[c].view(np.uint32), refs[c % distinct].view(np.uint32)), "column %d" % c
-    assert (kernels == ["cj_gemm_t_q4k"]) == tiled, kernels
+    assert kernels[0].startswith("cj_gemm_t_") == tiled, kernels
     for b in (w, src, xb, y):
         b.free()
 
