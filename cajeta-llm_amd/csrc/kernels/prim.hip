@@ -28,7 +28,9 @@ extern "C" __global__ void __launch_bounds__(256) cj_pack(cj_pack_args a) {
 // The pack alone, a wave a 256-wide block (four a workgroup, over all the
 // rows' blocks). Bound by latency at one row: a workgroup a row, as cj_pack,
 // walked a 14336-wide row's 56 blocks on one CU (with the Q4_K product after
-// it, 12.4 us a pass; 10.0 with this).
+// it, 12.4 us a pass; 10.0 with this). Many wide rows stay with cj_pack, whose
+// lanes hold 16 values and share the block's steps among fewer (512 rows of
+// 14336: 9.2 us here, 8.0 there).
 extern "C" __global__ void __launch_bounds__(256) cj_pack_blocks(cj_pack_args a) {
     const int lane = threadIdx.x & 63;
     const int64_t nblk = a.npad / 256, i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);

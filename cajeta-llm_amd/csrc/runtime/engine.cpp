@@ -922,11 +922,11 @@ int Engine::rows_norm_pack(const float *w, int per32, int n) {
     return launch_norm_pack_rows(a, n);
 }
 
-// The f32 rows x (n wide) packed into r_ap, a wave a 256-block.
+// The f32 rows x (n wide) packed into r_ap.
 int Engine::rows_pack(const float *x, int64_t n, int per32, int rows) {
     cj_pack_args p{};
     p.out = r_ap; p.x = x; p.n = n; p.npad = (n + 255) / 256 * 256; p.rows = rows; p.per32 = per32;
-    return launch("cj_pack_blocks", (uint32_t)((p.npad / 256 * rows + 3) / 4), 256, 0, p);
+    return launch_pack(p);
 }
 
 // Whether cj_rows_router takes n rows' router product. It is one chain of

@@ -58,6 +58,8 @@ int run_gemv(const cj_gemv_args &a, const GemvPlan &p);
 // floats apart); STORE or ACCUM epilogue.
 bool gemm_supported(int type);
 int run_gemm(const cj_gemv_args &a);
+// The pack of a.rows f32 rows, without a norm.
+int launch_pack(const cj_pack_args &a);
 
 // Device memory owned by the runtime itself (not through the handle table's
 // public free): allocation + registration for the extent checks.

@@ -811,3 +811,24 @@ def test_pack_rows_of_any_width(gpu, O, per32, rows, n, off):
     for r in range(rows):
         ref = O.q8k_pack(x[off + r * n:off + (r + 1) * n], per32=bool(per32), npad=npad)
         assert np.array_equal(got[r], ref), "row %d" % r
+
+
+@pytest.mark.parametrize("per32", [0, 1])
+@pytest.mark.parametrize("rows,n,off,kernel", [(384, 4096, 0, "cj_pack"), (383, 4096, 0, "cj_pack_blocks"), (1024, 1280, 0, "cj_pack"),
+                                               (1024, 1024, 0, "cj_pack_blocks"), (512, 2884, 0, "cj_pack"),
+                                               (512, 4096, 1, "cj_pack_blocks"), (512, 3001, 0, "cj_pack_blocks")])
+def test_pack_of_many_rows(gpu, O, launched, per32, rows, n, off, kernel):
+    """cj_q8k_pack on both sides of the line between a workgroup a row (many
+    wide aligned rows) and a wave a block; the same bytes."""
+    say("pack many rows", per32, rows, n, off)
+    rng = np.random.default_rng(rows * n + per32)
+    npad = (n + 255) // 256 * 256
+    x = rng.standard_normal(off + rows * n).astype(np.float32)
+    xb, ob = gpu.Buffer.of(x), gpu.Buffer(rows * npad // 256 * 320)
+    _, kernels = launched(lambda: gpu.native.check(
+        gpu.native.lib().cj_q8k_pack(ob.h, xb.h + 4 * off, rows, n, npad, per32), "pack"))
+    got = ob.download(np.uint8, rows * npad // 256 * 320).reshape(rows, -1)
+    for r in range(rows):
+        ref = O.q8k_pack(x[off + r * n:off + (r + 1) * n], per32=bool(per32), npad=npad)
+        assert np.array_equal(got[r], ref), "row %d" % r
+    assert kernels == [kernel]
