@@ -374,13 +374,16 @@ def test_prefill_attend_query_groups(gpu, heads, kv):
 
 
 @pytest.mark.parametrize("heads,kv,swa,chunk,n", [(8, 2, 40, 37, 150), (16, 2, 100, 19, 150), (4, 4, 7, 50, 120),
-                                                  (8, 4, 16, 2, 40), (8, 2, 0, 512, 15), (8, 2, 0, 512, 34)])
+                                                  (8, 4, 16, 2, 40), (8, 2, 0, 512, 15), (8, 2, 0, 512, 34),
+                                                  (8, 1, 0, 512, 3), (8, 1, 6, 3, 40), (8, 4, 0, 5, 13), (8, 8, 0, 512, 2),
+                                                  (8, 1, 20, 9, 45), (8, 2, 0, 512, 9)])
 def test_prefill_attend_runs(gpu, heads, kv, swa, chunk, n):
     """The prefill attend's runs of 16 positions off their edges: windows that
     start and chunks that end inside a run, rows of a wave that see different
-    positions, a prompt shorter than a run; bit for bit."""
+    positions, prompts shorter than a run (of which four positions at a time
+    are formed, up to the last one seen); bit for bit."""
     say("prefill attend runs", heads, kv, swa, chunk, n)
-    name = "t_pfr%d_%d_%d" % (heads, kv, chunk)
+    name = "t_pfr%d_%d_%d_%d" % (heads, kv, chunk, n)
     spec = "layers=2;hidden=1024;heads=%d;kv=%d;hd=128;ffn=1024;vocab=2048;eps=1e-5;theta=10000;" \
            "wtype=q8_0;head=q8_0;embd=q8_0;ctx=256%s" % (heads, kv, ";swa=%d" % swa if swa else "")
     path, img = synth(gpu, spec, name, 31 + n)
