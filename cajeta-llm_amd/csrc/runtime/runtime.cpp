@@ -64,8 +64,8 @@ const std::unordered_map<std::string, std::string> &name_map() {
         {"q40F32WaveMatVecKernel", "cj_gemv_q40b_r4"},
         {"mxfp4MatVecKernel", "cj_gemv_mxfp4"},
         {"mxfp4MatVecKernelCoopQ8", "cj_gemv_mxq8_s_k3_r4"},
-        {"q8kPackKernel", "cj_pack"},
-        {"q8kPack32Kernel", "cj_pack"},
+        {"q8kPackKernel", "cj_pack_blocks"},
+        {"q8kPack32Kernel", "cj_pack_blocks"},
         {"rmsnormPackRowF32", "cj_pack"},
         {"rmsnormRowF32", "cj_pack"},
         {"gluPackF32", "cj_glu"},
@@ -723,6 +723,7 @@ int32_t cj_event_free(int64_t ev) {
 
 int32_t cj_q8k_pack(int64_t out, int64_t x, int64_t rows, int64_t n, int64_t npad, int32_t per32) {
     if (rows <= 0 || n <= 0 || npad < n || npad % 256) return fail(CJ_ERR_ARG, "cj_q8k_pack: rows %lld n %lld npad %lld", (long long)rows, (long long)n, (long long)npad);
+    // (a workgroup a row stages the row's pack in LDS)
     if (npad / 256 > 64) return fail(CJ_ERR_ARG, "cj_q8k_pack: %lld columns exceed the 16384 staged", (long long)npad);
     if (!in_buffer(dptr(x), rows * n * 4) || !in_buffer(dptr(out), rows * npad / 256 * 320))
         return fail(CJ_ERR_ARG, "cj_q8k_pack: buffers smaller than %lld rows", (long long)rows);
@@ -904,7 +905,7 @@ int32_t cj_attend(int64_t part, int64_t out, int64_t q, int64_t kcache, int64_t 
     if (!in_buffer(dptr(pgtab + 4 * pg_base), pages * 4) || !in_buffer(dptr(q), (int64_t)n_q * head_dim * 4) ||
         !in_buffer(dptr(part), part_bytes) || (!split && !out) ||
         (out && !in_buffer(dptr(out), (int64_t)n_q * head_dim * 4)) ||
-        (split && out && !in_buffer(dptr(counters), (int64_t)n_kv * 4)))
+        (split && out && !in_buffer(dptr(counters), (int64_t)n_kv * 4)))   // (unused since the merge is a launch of its own)
         return fail(CJ_ERR_ARG, "cj_attend: a buffer is smaller than the shapes need");
     int32_t minpg = 0, maxpg = 0;
     if (int32_t rc = page_span(dptr(pgtab + 4 * pg_base), pages, minpg, maxpg)) return rc;

@@ -176,8 +176,9 @@ int32_t cj_qk_prep(int64_t q, int64_t k, int64_t v, int64_t kcache, int64_t vcac
  *  - head_dim 128 with 4 or 8 query heads per kv head: split-K into
  *    cj_decode_splits(count, n_kv, workers) splits, partials
  *    [n_q][64][hd+2] (acc, max, sum) into `part`; when out != 0 a
- *    second launch merges them into out [n_q·hd] (counters: n_kv int32
- *    words, zero before the call and left zero after). Replaces
+ *    second launch merges them into out [n_q·hd]. (counters: n_kv int32
+ *    words, required with out and checked for size; the merge being a
+ *    launch of its own, no kernel reads or writes them.) Replaces
  *    AttnKernel.attnDecodeCpuGqaKernel / cpuDecodeHead
  *    (model/AttnKernel.cajeta:4216-4314) behind
  *    attendDecodePartialsLaunchNoSync (:5090-5135) and, with out,
