@@ -683,9 +683,9 @@ def test_allocating_argmax_refuses_a_graph_capture(gpu):
                                              (40, 768, 30000), (16448, 1024, 33), (4160, 1312, 130),
                                              (1030, 32, 300)])
 def test_matmul_tile_kernels(gpu, O, name, ty, rows, cols, ncols):
-    """Shapes that take the 64-row × 128-column tile kernels (more tiles than
-    a CU's worth of the others'), off the tile's edges, one block to nine, and
-    for Q8_0 rows that end inside a 256-element group:
+    """Shapes around the 64-row × 128-column tile kernels (most take them),
+    off the tile's edges, one block to nine, and for Q8_0 rows that end inside
+    a 256-element group:
     every column checked bit for bit against the oracle's one-column product.
     Row 0 and column 0 hold the largest codes and scales, so their integer
     sums reach their bounds."""
@@ -723,6 +723,49 @@ def test_matmul_tile_kernels(gpu, O, name, ty, rows, cols, ncols):
     for c in range(ncols):
         assert np.array_equal(got[c].view(np.uint32), refs[c % distinct].view(np.uint32)), \
             "%s column %d: %d rows differ" % (name, c, int((got[c] != refs[c % distinct]).sum()))
+    for b in (w, src, xb, y):
+        b.free()
+
+
+@pytest.mark.parametrize("accum", [0, 1])
+@pytest.mark.parametrize("name,ty,rows,cols,ncols", [("q4k", 12, 4161, 1280, 129), ("q4k", 12, 16330, 1024, 150),
+                                                     ("q6k", 14, 2050, 2304, 300), ("q6k", 14, 16330, 1024, 150),
+                                                     ("q80", 8, 4161, 1312, 129), ("q80", 8, 16330, 1024, 150)])
+def test_matmul_tile_outputs(gpu, O, launched, name, ty, rows, cols, ncols, accum):
+    """The tile kernels in one round of tiles and in several, into outputs that
+    start at an offset and lie further apart than the rows: stored or added to
+    what stands there, bit for bit, with what lies between left alone. Rows 1
+    to 4 hold an infinite or NaN block scale."""
+    say("matmul tile outputs", name, rows, cols, ncols, accum)
+    rng = np.random.default_rng(rows + cols + ncols + accum)
+    be, bb = O.BLOCK[ty]
+    raw = rand_blocks(O, ty, rows * cols // be, rng).reshape(rows, cols // be, bb).copy()
+    at = 208 if ty == O.Q6_K else 0                 # the f16 block scale
+    for r, v in ((1, np.inf), (2, np.nan), (3, -np.inf)):
+        raw[r, -1, at:at + 2] = np.asarray([v], np.float16).view(np.uint8)
+    if ty == O.Q4_K:
+        raw[4, 0, 2:4] = np.asarray([np.inf], np.float16).view(np.uint8)
+    lib = gpu.native.lib()
+    w = gpu.Buffer(lib.cj_prepared_row_bytes(ty, cols) * rows)
+    src = gpu.Buffer.of(raw.reshape(-1))
+    gpu.native.check(lib.cj_prepare_weight(w.h, src.h, ty, rows, cols), "prepare")
+    distinct, npad = 5, (cols + 255) // 256 * 256   # later columns repeat them
+    packs = np.stack([O.q8k_pack(rng.standard_normal(cols).astype(np.float32), per32=(ty == O.Q8_0), npad=npad)
+                      for _ in range(distinct)])
+    refs = np.stack([O.matvec_packed(ty, raw.reshape(-1), rows, cols, p) for p in packs])[np.arange(ncols) % distinct]
+    y_off, y_stride = 3, rows + 10
+    y0 = rng.standard_normal((ncols, y_stride)).astype(np.float32)
+    xb, y = gpu.Buffer.of(packs[np.arange(ncols) % distinct].reshape(-1)), gpu.Buffer.of(y0)
+    _, kernels = launched(lambda: gpu.native.check(
+        lib.cj_matmul(ty, y.h, w.h, xb.h, rows, cols, ncols, packs.shape[1], y_stride, y_off, accum), "matmul"))
+    assert kernels == ["cj_gemm_t_" + name]
+    got = y.download(np.float32, ncols * y_stride).reshape(ncols, y_stride)
+    want = y0.copy()
+    with np.errstate(invalid="ignore"):
+        want[:, y_off:y_off + rows] = y0[:, y_off:y_off + rows] + refs if accum else refs
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isnan(want).any() and np.isinf(want).any()
+    same = (got.view(np.uint32) == want.view(np.uint32)) | np.isnan(want)
+    assert same.all(), "%d values differ" % int((~same).sum())
     for b in (w, src, xb, y):
         b.free()
 
@@ -793,6 +836,65 @@ def test_page_table_checks(gpu, O, pages):
             assert attend() == 0
             gpu.native.sync()
             bb.free()
+
+
+def test_page_table_check_behind_long_work(gpu, O):
+    """A check that is queued behind several milliseconds of products still
+    reads the table as the queued work leaves it, and refuses or accepts by it."""
+    import time
+    say("page table check behind long work")
+    lib = gpu.native.lib()
+    rows, cols, ncols = 14336, 4096, 512
+    w, xb = gpu.Buffer(lib.cj_prepared_row_bytes(O.Q8_0, cols) * rows), gpu.Buffer(ncols * cols // 256 * 320)
+    y = gpu.Buffer(ncols * rows * 4)
+    w.zero(); xb.zero()
+    nq, nkv, hd, pages = 2, 1, 64, 8
+    kc, vc = gpu.Buffer(nkv * 64 * hd * 2), gpu.Buffer(nkv * 64 * hd * 2)      # page 0 alone exists
+    kc.zero(); vc.zero()
+    q, out, part = gpu.Buffer(nq * hd * 4), gpu.Buffer(nq * hd * 4), gpu.Buffer(nq * pages * 64 * 4)
+    q.zero()
+    tab, good = gpu.Buffer(pages * 4), gpu.Buffer.of(np.zeros(pages, np.int32))
+    bad = gpu.Buffer.of(np.asarray([0, 0, 0, 0, 0, 0, 0, 1], np.int32))
+    for first, last, rc in ((good, bad, -1), (bad, good, 0)):
+        gpu.native.check(lib.cj_buf_copy(tab.h, first.h, pages * 4), "copy")
+        gpu.native.sync()
+        for _ in range(150):                         # each over 100 us
+            gpu.native.check(lib.cj_matmul(O.Q8_0, y.h, w.h, xb.h, rows, cols, ncols, cols // 256 * 320, rows, 0, 0), "matmul")
+        gpu.native.check(lib.cj_buf_copy(tab.h, last.h, pages * 4), "copy")
+        t = time.perf_counter()
+        assert lib.cj_attend(part.h, out.h, q.h, kc.h, vc.h, tab.h, 0, 0, nq, nkv, hd, pages * 64, 0, 512, 0.125) == rc
+        assert time.perf_counter() - t > 0.005       # it did wait: longer than the word is polled for
+        gpu.native.sync()
+    for b in (w, xb, y):
+        b.free()
+
+
+def test_page_table_checks_of_two_threads(gpu, O):
+    """Attends from two threads, one over good tables and one over bad ones:
+    each gets the answer to its own table."""
+    import threading
+    say("page table checks of two threads")
+    lib = gpu.native.lib()
+    nq, nkv, hd, pages = 2, 1, 64, 5
+    kc, vc = gpu.Buffer(nkv * 64 * hd * 2), gpu.Buffer(nkv * 64 * hd * 2)
+    kc.zero(); vc.zero()
+    q = gpu.Buffer(nq * hd * 4)
+    q.zero()
+    answers = {0: [], 1: []}
+
+    def attend(page):
+        tab = gpu.Buffer.of(np.asarray([0, 0, page, 0, 0, 0, 0, 0], np.int32))
+        out, part = gpu.Buffer(nq * hd * 4), gpu.Buffer(nq * pages * 64 * 4)
+        for _ in range(200):
+            answers[page].append(lib.cj_attend(part.h, out.h, q.h, kc.h, vc.h, tab.h, 0, 0, nq, nkv, hd, pages * 64, 0, 512, 0.125))
+        gpu.native.sync()
+
+    threads = [threading.Thread(target=attend, args=(p,)) for p in (0, 1)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert answers == {0: [0] * 200, 1: [-1] * 200}
 
 
 @pytest.mark.parametrize("per32", [0, 1])

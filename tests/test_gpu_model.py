@@ -425,12 +425,13 @@ def test_c4_shape_q8_0_batched_decode_parity(gpu):
 
 
 @pytest.mark.parametrize("hidden,ffn,experts,used,n", [(512, 1056, 4, 2, 150), (2080, 512, 2, 1, 66), (1024, 2112, 3, 3, 33),
-                                                       (512, 32, 5, 2, 90)])
-def test_moe_expert_tiles(gpu, hidden, ffn, experts, used, n):
-    """MXFP4 experts of a prefill chunk on the matrix-core tiles: rows of one
-    to three sweeps of 32 blocks, ones that end inside a sweep and inside a
-    pack block among them, and members on either side of a chunk of 32; bit
-    for bit."""
+                                                       (512, 32, 5, 2, 90), (1056, 96, 2, 1, 80), (1568, 1056, 3, 2, 70),
+                                                       (2048, 1024, 2, 2, 33)])
+def test_moe_expert_tiles(gpu, launched, hidden, ffn, experts, used, n):
+    """MXFP4 experts of a prefill chunk on the matrix-core tiles: gate|up and
+    down rows of one to three sweeps of 32 blocks, ones that end inside a sweep
+    and inside a pack block among them, and members on either side of a chunk
+    of 32; bit for bit."""
     say("moe expert tiles", hidden, ffn, experts, used, n)
     name = "t_moet%d_%d" % (hidden, ffn)
     spec = "layers=2;hidden=%d;heads=8;kv=2;hd=64;ffn=%d;vocab=2048;eps=1e-5;theta=150000;wtype=q8_0;head=q8_0;embd=q8_0;" \
@@ -438,10 +439,12 @@ def test_moe_expert_tiles(gpu, hidden, ffn, experts, used, n):
     path, img = synth(gpu, spec, name, 7 + n)
     rng = np.random.default_rng(hidden + n)
     prompt = rng.integers(0, 2048, n).tolist()
-    g, o, err = run_pair(gpu, path, img, prompt, 2, 256)
+    (g, o, err), kernels = launched(lambda: run_pair(gpu, path, img, prompt, 2, 256))
     gpu.image_free(name)
     assert g == o
     assert run_pair.bit_identical, err
+    sweeps = [(c + 1023) // 1024 for c in (hidden, ffn)]
+    assert "cj_moe_t_g_k%d" % sweeps[0] in kernels and "cj_moe_t_s_k%d" % sweeps[1] in kernels, kernels
 
 
 @pytest.mark.parametrize("hidden,experts,used,n,etype,tiled", [(2080, 8, 2, 64, "mxfp4", False), (512, 4, 2, 64, "q8_0", False),
