@@ -3,7 +3,10 @@
 // the int8 matrix cores, bit for bit what the one-column GEMV gives each
 // column (gemm.hip states the reference's order for each format).
 //
-// What bounds a product of this shape is VALU issue, not the matrix cores:
+// What bounds a full product of this shape is VALU issue, not the matrix cores
+// (counters: Q4_K 89% of the SIMD cycles against 13%, Q8_0 78% against 21%;
+// Q6_K, which folds its scales at staging, 49% against 25% on the CUs with a
+// tile):
 // the integer sub-block sums become f32 through arithmetic that the
 // reference's order fixes per output. Measured here: an f32 multiply, add or
 // fma issues in 2.5 cycles with two waves on a SIMD (5 with one), a
@@ -668,12 +671,15 @@ extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_pe
 // the members, which go 32 a chunk; the next chunk's codes are requested
 // before the current one's epilogue.
 //
-// Bound by VALU issue: four steps an output and block (the sum's conversion,
-// the two scales, the add), where the dot4 kernel spends twelve.
+// VALU issue takes 55% of the SIMD cycles (counters, 300 rows, gate|up; matrix
+// cores 4%): four steps an output and block (the sum's conversion, the two
+// scales, the add), where the dot4 kernel spends twelve; a third of the wave
+// cycles wait at two waves a SIMD.
 // Measured (MI355X, 32 experts of 2880 × 2880, 4 a row): 512 rows gate|up
-// 1056 → 459 us, down 598 → 276; 128 rows 322 → 270, 186 → 155. At few rows
-// the weights' decode and scale table (about 150 us for all the experts)
-// bound it.
+// 1058 → 449 us, down 604 → 261; 128 rows 281 → 263, 163 → 140. One and two
+// sweeps: 8 experts of 2048 × 1024, 2 a row, 64 rows 38 → 15 and 18 → 8. At
+// few rows the weights' decode and scale table bound it (2880 × 2880: 250 us
+// and 124 for all the experts from 24 to 64 rows).
 template <int EPI, int KB>
 DEV void moe_tile_body(const cj_moe_grp_args &a) {
     constexpr int RT = EPI == CJ_EPI_GLU ? 2 : 1, ROWS = 32 * RT, NM = 4 * KB, WS = ROWS + 4;

@@ -998,9 +998,13 @@ int Engine::rows_moe(const Layer &L, int n) {
             const int nbq = (int)(q.cols / 32), kb = std::min(4, std::max(1, (nbq + 31) / 32));
             // the matrix-core tiles from 14 selections an expert on, and where
             // a wave's decoded rows fit its registers (96 blocks). Measured
-            // (32 experts of 2880, 4 a row; dot4 kernel → tiles, gate|up + down,
-            // us): 64 rows 282 → 367, 96 rows 397 → 384, 128 rows 508 → 425,
-            // 300 rows 1062 → 550, 512 rows 1653 → 735
+            // (us, dot4 kernel → tiles, gate|up + down): 32 experts of 2880 ×
+            // 2880, 4 a row: 96 rows 355 → 392, 112 rows (14 an expert) 411 →
+            // 406, 128 rows 444 → 403, 512 rows 1662 → 710; 64 of 2048 × 1408,
+            // 6 a row: 128 rows (12) 233 → 245, 192 rows 350 → 259; 128 of
+            // 2048 × 768, 8 a row: 192 rows (12) 231 → 231, 256 rows 307 → 239;
+            // 256 of 2048 × 512, 8 a row: 448 rows (14) 401 → 375. Few experts
+            // of few columns cross earlier (8 of 2048 × 1024: at 4)
             if (kb <= 3 && sels >= 14 * n_experts) {
                 char tname[32];
                 snprintf(tname, sizeof tname, "cj_moe_t_%s_k%d", form, kb);
